@@ -108,7 +108,7 @@ struct SysDesc {
   int NR, TXy, TXz;        // FFT tiles
   SolveArgs sa;            // influence function; sa.partial = this system's partials
   int nzblk;               // z-pass tiles (= partial count)
-  int plane;               // 1: x and y passes as one xy plane kernel
+  int plane;               // PLANE_*: how the x and y passes run
   void* force;             // caller's force output
   int force_type, stride;
   double* ev_out;          // [kEvOut]: energy, virial[9], self energy of the last solve (assigned)
@@ -116,6 +116,9 @@ struct SysDesc {
   int calc_self;           // 1: self energy (CudaPMERecip.cu:2053-2061)
   double kcs;              // kappa*ccelec/sqrt(pi)
 };
+// x and y passes: separate kernels, one xy plane kernel in Stockham or
+// matrix-core stages (two LDS buffers), or as register four-steps (one buffer)
+enum PlaneKind { PLANE_NONE = 0, PLANE_STAGES = 1, PLANE_FOUR_STEP = 2 };
 constexpr int kEvOut = 11;  // doubles per system in the batched energy/virial output
 
 // One workgroup-sized task of a batched stage: system index and the tile of
@@ -298,6 +301,37 @@ __device__ __forceinline__ void ev_reduce_block(const EvReduce& r) {
   }
 }
 
+// energy/virial of one system from its z-pass partials and its self energy
+// from the binning's per-chunk sums of q*q (fixed order, one workgroup),
+// assigned to ev_out
+template <int NT = kBlock>
+__device__ __forceinline__ void batch_ev_reduce(const SysDesc& d) {
+  __shared__ double sh[7 * (NT / 64)];
+  if (d.sa.calc_ev) {
+    double v[7] = {0, 0, 0, 0, 0, 0, 0};
+    for (int i = threadIdx.x; i < d.nzblk; i += NT)
+#pragma unroll
+      for (int c = 0; c < 7; c++) v[c] += d.sa.partial[(size_t)i * 7 + c];
+    block_sum<7, NT>(v, sh);
+    if (threadIdx.x == 0) {
+      const double hc = 0.5 * kCcelec;
+      double* o = d.ev_out;
+      o[0] = v[0] * hc;
+      const double v0 = -hc * v[1], v1 = -hc * v[2], v2 = -hc * v[3];
+      const double v3 = -hc * v[4], v4 = -hc * v[5], v5 = -hc * v[6];
+      o[1] = v0; o[2] = v1; o[3] = v2;
+      o[4] = v1; o[5] = v3; o[6] = v4;
+      o[7] = v2; o[8] = v4; o[9] = v5;
+    }
+  }
+  if (d.calc_self) {
+    double v[1] = {0.0};
+    for (int i = threadIdx.x; i < d.bin.nchunk; i += NT) v[0] += d.self_partial[i];
+    block_sum<1, NT>(v, sh);
+    if (threadIdx.x == 0) d.ev_out[10] = -v[0] * d.kcs;
+  }
+}
+
 // xy plane kernels (x and y passes of one z plane in one workgroup):
 // forward reads the real plane and writes its half-spectrum plane, inverse
 // the reverse; a pending energy/virial reduction runs in one extra
@@ -334,6 +368,21 @@ bool plane_fits_half(int nx, int ny, int nf_x);
 // workgroup (two workgroups per CU), for systems with plane_fits_half only.
 hipError_t launch_batch_plane(int inverse, int reduce, int maxnp, int split, int half, const SysDesc* sys,
                               const WorkItem* items, int nitems, int grid, size_t lds, hipStream_t s);
+
+// Plane kernels as register four-steps (pme_plane.hip): both lengths have a
+// four-step pair (plane4_ok) and FP32 axes.
+bool plane4_ok(const RadixPlan& rx, const RadixPlan& ry);
+size_t fft_plane4_lds_bytes(int nx, int ny, int np);  // 0: does not fit one workgroup
+int plane4_group_host(int nx, int ny, int maxnp, bool half);
+bool plane4_fits_half(int nx, int ny);
+hipError_t launch_plane4_fwd(const float* grid, float2* cg, int nx, int ny, int nz, const AxisArgs& ax,
+                             const AxisArgs& ay, hipStream_t s);
+hipError_t launch_plane4_inv(const float2* cg, float* grid, int nx, int ny, int nz, const AxisArgs& ax,
+                             const AxisArgs& ay, const EvReduce& red, hipStream_t s);
+hipError_t launch_batch_plane4(int inverse, int reduce, int maxnp, int half, const SysDesc* sys, const WorkItem* items,
+                               int nitems, int grid, size_t lds, hipStream_t s);
+// how the x and y passes of a grid run (y_prec: PREC_* of the y axis)
+PlaneKind plane_kind(int nx, int ny, const RadixPlan& rx, const RadixPlan& ry, int y_prec);
 
 // batched launchers: `grid` persistent workgroups loop over the work items
 hipError_t launch_batch_bin(const SysDesc* sys, const WorkItem* items, int nitems, int grid, size_t lds, hipStream_t s);

@@ -53,10 +53,10 @@ static void pack_radices(RadixPlan* rp) {
 }
 
 // Factor pair of the register four-step transform: n = a * b with both
-// codelet lengths (2, 3, 4, 5, 6, 8, 9, 10, 12, 16), the most balanced such
+// codelet lengths (2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16), the most balanced such
 // pair; (0, 0) when there is none.
 static void four_step_factors(int n, int* fa, int* fb) {
-  static const int L[] = {2, 3, 4, 5, 6, 8, 9, 10, 12, 16};
+  static const int L[] = {2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16};
   *fa = *fb = 0;
   int best = 1 << 30;
   for (int a : L)

@@ -56,7 +56,7 @@ pme_status plan_system(const pme_system_desc& in, int cap_atoms, const Tuning& t
   }
   p->ft = pick_fft_tiles(n[0], n[1], n[2], p->rp[0].n, t.fft_tile,
                          p->prec[2] == PME_PREC_FP32 && four_step_code(n[2]) >= 0);
-  p->plane = fft_plane_lds_bytes(n[0], n[1], p->rp[0].n, 1) != 0 ? 1 : 0;
+  p->plane = plane_kind(n[0], n[1], p->rp[0], p->rp[1], p->prec[1]);
   const int hx = n[0] / 2 + 1;
   if (p->ft.TXz <= 0 || (p->ft.TXz & (p->ft.TXz - 1)) != 0)  // the z pass indexes its tiles with shifts
     return set_error(PME_ERR_UNSUPPORTED, "system: z tile %d is not a power of two", p->ft.TXz);
@@ -201,7 +201,7 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
   // items per CU.
   int total_planes = 0;
   for (int k = 0; k < n; k++)
-    if (descs[k]->plane) total_planes += descs[k]->bin.nz;
+    if (descs[k]->plane != PLANE_NONE) total_planes += descs[k]->bin.nz;
   int group = kPlaneGroupMax;
   while (group > 1 && total_planes < 2 * ncu * group) group--;
   // order: the spread/gather order, or the largest plane group of a plane launch
@@ -216,7 +216,8 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
       const SysDesc& d = *descs[k];
       const SystemPlan& p = *plans[k];
       if ((stage == BS_SPREAD || stage == BS_GATHER) && orders[k] != order) continue;
-      if (stage == BS_FFTY || stage == BS_PLANE || stage == BS_FFTZ) {
+      if (stage == BS_PLANE && (d.plane == PLANE_FOUR_STEP) != (split == 2)) continue;
+      if (stage == BS_FFTY || (stage == BS_PLANE && split != 2) || stage == BS_FFTZ) {
         const int a = stage == BS_FFTZ ? 2 : 1;
         if ((d.ax[a].prec != PME_PREC_FP32) != (split != 0)) continue;
       }
@@ -240,19 +241,22 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
           lds = gather_lds_bytes(orders[k], p.bp.wmax, d.bin.nchunk);
           break;
         case BS_FFTX:
-          if (d.plane) break;
+          if (d.plane != PLANE_NONE) break;
           cnt = (d.bin.ny * d.bin.nz + d.NR - 1) / d.NR;
           lds = fft_x_lds_bytes(d.ax[0].rp.n, d.NR, d.bin.nx);
           break;
         case BS_FFTY:
-          if (d.plane) break;
+          if (d.plane != PLANE_NONE) break;
           cnt = cols_blocks(hx, d.TXy, d.bin.nz);
           lds = fft_cols_lds_bytes(d.bin.ny, d.TXy);
           break;
         case BS_PLANE: {
-          if (!d.plane || plane_fits_half(d.bin.nx, d.bin.ny, d.ax[0].rp.n) != (half != 0)) break;
-          const int g = plane_group_host(d.bin.nx, d.bin.ny, d.ax[0].rp.n, order, half != 0);
-          lds = fft_plane_lds_bytes(d.bin.nx, d.bin.ny, d.ax[0].rp.n, g);
+          if (d.plane == PLANE_NONE) break;
+          const bool f4 = d.plane == PLANE_FOUR_STEP;
+          const int nx = d.bin.nx, ny = d.bin.ny, nf = d.ax[0].rp.n;
+          if ((f4 ? plane4_fits_half(nx, ny) : plane_fits_half(nx, ny, nf)) != (half != 0)) break;
+          const int g = f4 ? plane4_group_host(nx, ny, order, half != 0) : plane_group_host(nx, ny, nf, order, half != 0);
+          lds = f4 ? fft_plane4_lds_bytes(nx, ny, g) : fft_plane_lds_bytes(nx, ny, nf, g);
           for (int z = 0; z < d.bin.nz; z += g) items.push_back(WorkItem{k, z});
           L.count += (d.bin.nz + g - 1) / g;
           break;
@@ -272,7 +276,7 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
   for (int o : {4, 6, 8}) add_stage(BS_SPREAD, o, 0, 0);
   add_stage(BS_FFTX, 0, 0, 0);
   for (int sp : {0, 1}) add_stage(BS_FFTY, 0, sp, 0);
-  for (int sp : {0, 1})
+  for (int sp : {0, 1, 2})
     for (int h : {1, 0}) add_stage(BS_PLANE, group, sp, h);
   for (int c : {1, 2}) add_stage(BS_FFTZ, c, 0, 0);
   for (int sp : {0, 1}) add_stage(BS_FFTZ, 0, sp, 0);
@@ -331,6 +335,11 @@ pme_status enqueue_stages(const std::vector<Launch>& launches, const SysDesc* d_
                                         stream));
             break;
           case BS_PLANE:
+            if (L.split == 2) {
+              SCHED_HIP(launch_batch_plane4(inv ? 1 : 0, inv ? 1 : 0, L.order, L.half, d_sys, it, L.count, grid, L.lds,
+                                            stream));
+              break;
+            }
             SCHED_HIP(launch_batch_plane(inv ? 1 : 0, inv ? 1 : 0, L.order, L.split, L.half, d_sys, it, L.count, grid, L.lds,
                                          stream));
             break;

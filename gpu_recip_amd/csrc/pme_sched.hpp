@@ -25,7 +25,7 @@ struct SystemPlan {
   int prec[3];          // PREC_* per axis (the radix-16 stage on the matrix cores)
   FftTiles ft;
   int nzblk;            // z-pass tiles = energy/virial partials
-  int plane;            // 1: x and y passes as one xy plane kernel
+  int plane;            // PLANE_*: how the x and y passes run
   size_t off[7];        // grid, cgrid, seg_off, rec_pos, rec_idx, partial, self_partial
   size_t total;         // bytes of the region
 };
@@ -74,7 +74,8 @@ struct Launch {
   int stage;   // BatchStage
   int order;   // spread/gather template order; largest plane group of a plane launch; z pass: 1 + the
                // four-step register class, 0 for the Stockham / split kernels (0 otherwise)
-  int split;   // FFT launches: 1 for the kernels with the split-precision matrix-core stage
+  int split;   // FFT launches: 1 for the kernels with the split-precision matrix-core stage; plane
+               // launches: 2 for the register four-step planes
   int half;    // plane launches: 1 for half-size workgroups (two per CU)
   int offset;
   int count;
