@@ -86,7 +86,6 @@ struct pme_batch_s {
   std::vector<Launch> launches_aux[kMaxBatchChains - 1];  // chain c on aux[c - 1] (empty: unused)
   hipStream_t aux[kMaxBatchChains - 1] = {};
   hipEvent_t ev_fork = nullptr, ev_join[kMaxBatchChains - 1] = {};
-  int* d_ctr = nullptr;  // work-queue counters: 2 per launch, chain c at c * 2 * kMaxLaunches
   WorkItem* d_items = nullptr;
   size_t items_cap = 0;
   // graph of the current subset
@@ -189,15 +188,13 @@ extern "C" pme_status pme_batch_create(size_t hbm_budget_bytes, pme_stream_t str
     }
     b->own_stream = true;
   }
-  bool ok = hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) == hipSuccess &&
-            hipMalloc(&b->d_ctr, sizeof(int) * 2 * kMaxLaunches * kMaxBatchChains) == hipSuccess &&
-            hipMemset(b->d_ctr, 0, sizeof(int) * 2 * kMaxLaunches * kMaxBatchChains) == hipSuccess;
+  bool ok = hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) == hipSuccess;
   for (int c = 0; ok && c < kMaxBatchChains - 1; c++)
     ok = hipStreamCreateWithFlags(&b->aux[c], hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&b->ev_join[c], hipEventDisableTiming) == hipSuccess;
   if (!ok) {
     pme_batch_destroy(b);
-    return set_error(PME_ERR_DEVICE, "pme_batch_create: auxiliary streams, events or work-queue counters failed");
+    return set_error(PME_ERR_DEVICE, "pme_batch_create: auxiliary streams or events failed");
   }
   int dev = 0;
   hipDeviceProp_t prop;
@@ -227,7 +224,6 @@ extern "C" pme_status pme_batch_destroy(pme_batch_t b) {
   (void)hipFree(b->d_ev);
   (void)hipHostFree(b->h_ev);
   (void)hipFree(b->d_items);
-  (void)hipFree(b->d_ctr);
   for (hipEvent_t e : b->tev)
     if (e) (void)hipEventDestroy(e);
   if (b->ev_in) (void)hipEventDestroy(b->ev_in);
@@ -367,16 +363,15 @@ static pme_status enqueue(pme_batch_t b) {
     BHIP(hipEventRecord(b->ev_fork, b->stream));
     for (int c = 1; c < kMaxBatchChains; c++)
       if (!b->launches_aux[c - 1].empty()) BHIP(hipStreamWaitEvent(b->aux[c - 1], b->ev_fork, 0));
-    BTRY(enqueue_stages(b->launches, b->d_sys, b->d_items, b->d_ctr, b->tune, b->ncu, b->stream, nullptr));
+    BTRY(enqueue_stages(b->launches, b->d_sys, b->d_items, b->tune, b->ncu, b->stream, nullptr));
     for (int c = 1; c < kMaxBatchChains; c++) {
       if (b->launches_aux[c - 1].empty()) continue;
-      BTRY(enqueue_stages(b->launches_aux[c - 1], b->d_sys, b->d_items, b->d_ctr + 2 * kMaxLaunches * c, b->tune,
-                          b->ncu, b->aux[c - 1], nullptr));
+      BTRY(enqueue_stages(b->launches_aux[c - 1], b->d_sys, b->d_items, b->tune, b->ncu, b->aux[c - 1], nullptr));
       BHIP(hipEventRecord(b->ev_join[c - 1], b->aux[c - 1]));
       BHIP(hipStreamWaitEvent(b->stream, b->ev_join[c - 1], 0));
     }
   } else {
-    BTRY(enqueue_stages(b->launches, b->d_sys, b->d_items, b->d_ctr, b->tune, b->ncu, b->stream,
+    BTRY(enqueue_stages(b->launches, b->d_sys, b->d_items, b->tune, b->ncu, b->stream,
                         b->timing ? b->tev : nullptr));
   }
   const int n = (int)b->slots.size();

@@ -122,9 +122,12 @@ __device__ __forceinline__ unsigned long long to_fixed_product(double a, double 
   const double t = __fma_rn(a, b, 6755399441055744.0);
   return (unsigned long long)__double_as_longlong(t) - 0x4338000000000000ull;
 }
-// back to FP32: ((float)val)*2^-40 as reduce_force<long long, float> (reduce.cu:66-78)
+// back to FP32: ((float)val)*2^-40 as reduce_force<long long, float>
+// (reduce.cu:66-78); the two halves are exact in FP64 and one FMA rounds their
+// sum, as the conversion of the 64-bit integer would
 __device__ __forceinline__ float from_fixed40(unsigned long long u) {
-  return (float)((double)(long long)u * (1.0 / 1099511627776.0));
+  const double lo = (double)(unsigned)u * (1.0 / 1099511627776.0);
+  return (float)__fma_rn((double)(int)(u >> 32), 1.0 / 256.0, lo);
 }
 
 // Brick decomposition of one grid axis into nb nearly equal bricks:

@@ -129,7 +129,9 @@ __device__ __forceinline__ void gather_atom(const BinArgs& a, const float4& p, i
 // that bin and gather the same coordinates (the batched path: one solve reads
 // the caller's array once).  Otherwise the current coordinates are read, so
 // an atom moved since the binning is still right (gather_atom).
-template <int P, bool FROM_REC, int NT>
+// STAGE: halo loads in flight per thread (a column of the halo brick in one
+// round up to STAGE planes).
+template <int P, bool FROM_REC, int NT, int STAGE>
 __device__ __forceinline__ void gather_brick_body(const float4* __restrict__ xyzq, const BinArgs& a, int b, int wxm,
                                                   int wym, int wzm, const float* __restrict__ phi, float ccelec_f,
                                                   int ft, int stride, void* force, unsigned char* smem) {
@@ -150,7 +152,7 @@ __device__ __forceinline__ void gather_brick_body(const float4* __restrict__ xyz
 
   // stage brick + upper halo (periodic) in LDS in this brick's own [hz][hy][hx]
   // layout: thread c takes column (lx, ly) = (c mod hx, c / hx) of the halo
-  // brick and walks it in z, kGatherStageU loads in flight (one division per
+  // brick and walks it in z, STAGE loads in flight (one division per
   // thread; consecutive threads read consecutive x, as rows of the grid)
   const int hx = wx + P - 1, hy = wy + P - 1, hz = wz + P - 1;
   const int ncol = hx * hy;
@@ -162,10 +164,10 @@ __device__ __forceinline__ void gather_brick_body(const float4* __restrict__ xyz
     if (gx >= a.nx) gx -= a.nx;
     if (gy >= a.ny) gy -= a.ny;
     const float* col = phi + (gx + mul24(a.nx, gy));
-    for (int lz0 = 0; lz0 < hz; lz0 += kGatherStageU) {
-      float v[kGatherStageU];
+    for (int lz0 = 0; lz0 < hz; lz0 += STAGE) {
+      float v[STAGE];
 #pragma unroll
-      for (int u = 0; u < kGatherStageU; u++) {
+      for (int u = 0; u < STAGE; u++) {
         // z0 + lz < nz + P - 1 < 2 nz for lz < hz: one wrap; 0 past the halo
         const int lz = lz0 + u;
         int gz = z0 + lz;
@@ -173,7 +175,7 @@ __device__ __forceinline__ void gather_brick_body(const float4* __restrict__ xyz
         v[u] = lz < hz ? col[mul24(nxny, lz < hz ? gz : 0)] : 0.f;
       }
 #pragma unroll
-      for (int u = 0; u < kGatherStageU; u++)
+      for (int u = 0; u < STAGE; u++)
         if (lz0 + u < hz) pl[mul24(lz0 + u, ncol) + c] = v[u];
     }
   }
@@ -207,13 +209,17 @@ __device__ __forceinline__ void gather_brick_body(const float4* __restrict__ xyz
   }
 }
 
-template <int P>
-__global__ __launch_bounds__(kSpreadBlock) void k_gather_brick(const float4* __restrict__ xyzq, BinArgs a, int wxm,
+// One workgroup per brick.  NT = 1024 when there are no more bricks than CUs;
+// NT = 512 when there are: two or three bricks then share a CU and one's
+// loads overlap the other's sums (400k atoms, 160^3, order 6, 512 bricks: 42.2
+// -> 33.0 us; with 252 bricks, one per CU, 14.8 against 17.0 us).
+template <int P, int NT>
+__global__ __launch_bounds__(NT, 4) void k_gather_brick(const float4* __restrict__ xyzq, BinArgs a, int wxm,
                                                                int wym, int wzm, const float* __restrict__ phi,
                                                                float ccelec_f, int ft, int stride, void* force) {
   extern __shared__ __align__(16) unsigned char smem[];
-  gather_brick_body<P, false, kSpreadBlock>(xyzq, a, blockIdx.x, wxm, wym, wzm, phi, ccelec_f, ft, stride, force,
-                                            smem);
+  gather_brick_body<P, false, NT, 24>(xyzq, a, xcd_brick(blockIdx.x, gridDim.x), wxm, wym, wzm, phi, ccelec_f,
+                                            ft, stride, force, smem);
 }
 
 size_t gather_lds_bytes(int order, const int wmax[3], int nchunk) {
@@ -223,52 +229,54 @@ size_t gather_lds_bytes(int order, const int wmax[3], int nchunk) {
 
 template <int P>
 static hipError_t launch_gather_p(int ft, const float4* xyzq, const BinArgs& a, const int wmax[3], const float* phi,
-                                  int stride, void* force, hipStream_t s) {
+                                  int stride, void* force, int ncu, hipStream_t s) {
   const int nbins = a.nbx * a.nby * a.nbz;
   const size_t lds = gather_lds_bytes(P, wmax, a.nchunk);
-  hipLaunchKernelGGL(k_gather_brick<P>, dim3(nbins), dim3(kSpreadBlock), lds, s, xyzq, a, wmax[0], wmax[1], wmax[2], phi,
-                     (float)kCcelec, ft, stride, force);
+  constexpr int H = kSpreadBlock / 2;
+  if (nbins > ncu)
+    hipLaunchKernelGGL((k_gather_brick<P, H>), dim3(nbins), dim3(H), lds, s, xyzq, a, wmax[0], wmax[1], wmax[2], phi,
+                       (float)kCcelec, ft, stride, force);
+  else
+    hipLaunchKernelGGL((k_gather_brick<P, kSpreadBlock>), dim3(nbins), dim3(kSpreadBlock), lds, s, xyzq, a, wmax[0],
+                       wmax[1], wmax[2], phi, (float)kCcelec, ft, stride, force);
   return hipGetLastError();
 }
 
 hipError_t launch_gather(int order, int force_type, const float4* xyzq, const BinArgs& a, const int wmax[3],
-                         const float* phi, int stride, void* force, hipStream_t s) {
+                         const float* phi, int stride, void* force, int ncu, hipStream_t s) {
   switch (order) {
-    case 4: return launch_gather_p<4>(force_type, xyzq, a, wmax, phi, stride, force, s);
-    case 6: return launch_gather_p<6>(force_type, xyzq, a, wmax, phi, stride, force, s);
-    case 8: return launch_gather_p<8>(force_type, xyzq, a, wmax, phi, stride, force, s);
+    case 4: return launch_gather_p<4>(force_type, xyzq, a, wmax, phi, stride, force, ncu, s);
+    case 6: return launch_gather_p<6>(force_type, xyzq, a, wmax, phi, stride, force, ncu, s);
+    case 8: return launch_gather_p<8>(force_type, xyzq, a, wmax, phi, stride, force, ncu, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-// ---- batched: persistent workgroups over the work items of many systems ----
+// ---- batched: the work items of many systems -----------------------------------
 
-// NT = kSpreadBlock / 2: half-size workgroups, two per CU, for bricks
-// planned within half the LDS budget (four waves per SIMD: at most 128 VGPRs)
+// NT = kSpreadBlock / 2: half-size workgroups for bricks planned within half the
+// LDS budget.  The gather's halo brick is about half of the spread's, so three
+// share a CU when the registers allow (12 instead of 24 halo loads in flight:
+// 80 VGPRs at order 4): 64-system set 46.1 -> 40.8 us.
 template <int P, int NT>
-__global__ __launch_bounds__(NT, 4) void k_batch_gather(const SysDesc* __restrict__ sys,
-                                                     const WorkItem* __restrict__ items, int nitems, int* ctr) {
+__global__ __launch_bounds__(NT, NT < kSpreadBlock && P < 8 ? 6 : 4) void k_batch_gather(const SysDesc* __restrict__ sys,
+                                                     const WorkItem* __restrict__ items) {
   extern __shared__ __align__(16) unsigned char smem[];
-  for (int it = blockIdx.x; it < nitems; it = next_item(nitems, ctr)) {
-    const WorkItem w = uniform_item(items[it]);
-    const SysDesc& d = sys[w.sys];
-    gather_brick_body<P, true, NT>(d.xyzq, d.bin, w.idx, d.wmax[0], d.wmax[1], d.wmax[2], d.grid, (float)kCcelec, d.force_type,
-                         d.stride, d.force, smem);
-    __syncthreads();
-  }
-  items_done(nitems, ctr);
+  const WorkItem w = uniform_item(items[blockIdx.x]);
+  const SysDesc& d = sys[w.sys];
+  gather_brick_body<P, true, NT, (NT < kSpreadBlock ? 12 : 24)>(d.xyzq, d.bin, w.idx, d.wmax[0], d.wmax[1], d.wmax[2], d.grid, (float)kCcelec,
+                                 d.force_type, d.stride, d.force, smem);
 }
 
-hipError_t launch_batch_gather(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems, int* ctr,
-                               int grid, size_t lds, hipStream_t s) {
+hipError_t launch_batch_gather(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems,
+                               size_t lds, hipStream_t s) {
   if (nitems <= 0) return hipSuccess;
   constexpr int H = kSpreadBlock / 2;
 #define PME_BGATHER(P)                                                                                           \
   if (half)                                                                                                      \
-    hipLaunchKernelGGL((k_batch_gather<P, H>), dim3(grid), dim3(H), lds, s, sys, items, nitems, ctr);            \
+    hipLaunchKernelGGL((k_batch_gather<P, H>), dim3(nitems), dim3(H), lds, s, sys, items);                       \
   else                                                                                                           \
-    hipLaunchKernelGGL((k_batch_gather<P, kSpreadBlock>), dim3(grid), dim3(kSpreadBlock), lds, s, sys, items,    \
-                       nitems, ctr);
+    hipLaunchKernelGGL((k_batch_gather<P, kSpreadBlock>), dim3(nitems), dim3(kSpreadBlock), lds, s, sys, items);
   switch (order) {
     case 4: PME_BGATHER(4) break;
     case 6: PME_BGATHER(6) break;

@@ -261,6 +261,7 @@ struct pme_recip_s {
 
   // bricks and the chunked record store of the binning
   int nb[3] = {1, 1, 1}, wmax[3] = {0, 0, 0}, nbins = 0;
+  int ncu = 256;              // compute units of the device
   int bins_for = -1;          // atom capacity of the record store
   int chunk = 0, nchunk = 0, nchunk_cap = 0;
   int* seg_off = nullptr;     // [nchunk_cap][seg_stride(nbins)]
@@ -364,11 +365,11 @@ static pme_status upload_prefac(pme_recip_t h) {
 static bool plan_bricks(pme_recip_t h) {
   const int n[3] = {h->nx, h->ny, h->nz};
   BrickPlan bp;
-  int dev = 0, ncu = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      ncu <= 0)
-    ncu = 256;
-  if (!pme::plan_bricks_auto(n, h->order, ncu, &bp)) return false;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || h->ncu <= 0)
+    h->ncu = 256;
+  if (!pme::plan_bricks_auto(n, h->order, h->ncu, &bp)) return false;
   for (int a = 0; a < 3; a++) {
     h->nb[a] = bp.nb[a];
     h->wmax[a] = bp.wmax[a];
@@ -782,7 +783,8 @@ extern "C" pme_status pme_recip_gather_force(pme_recip_t h, const void* d_xyzq, 
   }
   mark(h, 7);
   BinArgs a = bin_args(h, recip);
-  HIP_TRY(launch_gather(h->order, force_type, (const float4*)d_xyzq, a, h->wmax, h->grid, stride, d_force, h->stream));
+  HIP_TRY(launch_gather(h->order, force_type, (const float4*)d_xyzq, a, h->wmax, h->grid, stride, d_force,
+                        h->ncu, h->stream));
   mark(h, 8);
   return PME_OK;
 }

@@ -128,34 +128,6 @@ struct WorkItem {
   int idx;
 };
 
-// Work distribution of the batched spread and gather kernels (one brick per
-// item, one workgroup per CU at a time).  Workgroup b starts with item b.
-// With fewer workgroups than items (persistent launches) a workgroup that
-// finishes a brick takes the next one from the launch's counter ctr[0], so
-// the bricks balance as under the hardware dispatcher.  The fetch comes after
-// the brick's stores are issued and before the next brick's loads, since a
-// wait for those loads would also wait for an earlier fetch.  The last
-// workgroup to finish (counted in ctr[1]) puts both counters back to zero for
-// the next launch that uses them (stream order makes that launch see the
-// zeros).  One lane per workgroup touches the counters, with vector atomics.
-// The other batched kernels stride statically: their items are many and
-// short, and one counter shared by every XCD would serialize them.
-__device__ __forceinline__ int next_item(int nitems, int* ctr) {
-  if ((int)gridDim.x >= nitems) return nitems;
-  __shared__ int s_next;
-  __syncthreads();
-  if (threadIdx.x == 0) s_next = (int)gridDim.x + atomicAdd(&ctr[0], 1);
-  __syncthreads();
-  return s_next;
-}
-__device__ __forceinline__ void items_done(int nitems, int* ctr) {
-  if ((int)gridDim.x >= nitems) return;
-  if (threadIdx.x == 0 && atomicAdd(&ctr[1], 1) == (int)gridDim.x - 1) {
-    atomicExch(&ctr[0], 0);
-    atomicExch(&ctr[1], 0);
-  }
-}
-
 // Work items are the same for every lane of a workgroup: make that explicit
 // so descriptor fields are read with scalar loads and branch uniformly.
 __device__ __forceinline__ WorkItem uniform_item(WorkItem w) {
@@ -224,6 +196,15 @@ __device__ __forceinline__ int brick_segments(const BinArgs& a, const SegBounds&
   return total;
 }
 
+// Brick of workgroup blk of a launch with one workgroup per brick.  Workgroups
+// are dealt to the 8 XCDs in turn, each with its own L2; each XCD takes a
+// contiguous run of bricks, so the cache lines that x-neighbours share (rows of
+// a brick are short and unaligned) are merged in one L2.
+__device__ __forceinline__ int xcd_brick(int blk, int nbricks) {
+  const int x = blk & 7, per = nbricks >> 3, rem = nbricks & 7;
+  return x * per + min(x, rem) + (blk >> 3);
+}
+
 // record slot of the v-th record of the brick (0 <= v < total)
 __device__ __forceinline__ size_t brick_record(const BinArgs& a, int v, const int* s_pre, const int* s_base) {
   int lo = 0, hi = a.nchunk;  // s_pre[lo] <= v < s_pre[hi]
@@ -240,7 +221,7 @@ hipError_t launch_bin_atoms(const float4* xyzq, int n, const BinArgs& a, hipStre
 hipError_t launch_spread(int order, const BinArgs& a, const int wmax[3], float* grid, hipStream_t s);
 hipError_t launch_gather(int order, int force_type, const float4* xyzq, const BinArgs& a,
                          const int wmax[3], const float* phi, int stride, void* force,
-                         hipStream_t s);
+                         int ncu, hipStream_t s);
 
 // The half spectrum holds nz planes of pitch spec_pitch(hx, ny) complex
 // values, each plane ny rows of hx = nx/2 + 1 (kx fastest).
@@ -388,10 +369,10 @@ PlaneKind plane_kind(int nx, int ny, const RadixPlan& rx, const RadixPlan& ry, i
 hipError_t launch_batch_bin(const SysDesc* sys, const WorkItem* items, int nitems, int grid, size_t lds, hipStream_t s);
 // spread / gather: half != 0 runs kSpreadBlock / 2 threads per workgroup
 // (bricks planned within half the LDS budget, two workgroups per CU)
-hipError_t launch_batch_spread(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems, int* ctr,
-                               int grid, size_t lds, hipStream_t s);
-hipError_t launch_batch_gather(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems, int* ctr,
-                               int grid, size_t lds, hipStream_t s);
+hipError_t launch_batch_spread(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems,
+                               size_t lds, hipStream_t s);
+hipError_t launch_batch_gather(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems,
+                               size_t lds, hipStream_t s);
 hipError_t launch_batch_fft_x(int inverse, const SysDesc* sys, const WorkItem* items, int nitems, int grid, size_t lds,
                               hipStream_t s);
 // axis 1 (y) or 2 (z); mode COL_*; with reduce != 0 the first tile of every
@@ -414,7 +395,6 @@ size_t fft_cols_lds_bytes(int n, int TX, int nbuf = 2);
 
 constexpr int kSpreadBlock = 1024;  // threads per spread / gather workgroup (16 waves per CU)
 constexpr int kRecPerThread = 2;    // gather: brick records read per thread per round
-constexpr int kGatherStageU = 24;   // gather: halo loads in flight per thread (one round up to 24 K points)
 constexpr int kBinBlock = 512;     // threads per binning workgroup (one atom each at the default chunk)
 constexpr int kPlaneBlock = 1024;   // threads per xy plane FFT workgroup
 constexpr int kPlaneGroupMax = 4;   // z planes per batched plane workgroup (at most)

@@ -191,6 +191,21 @@ pme_status fill_desc(SysDesc& d, const pme_system_desc& in, const SystemPlan& p,
   return PME_OK;
 }
 
+// The bricks of system k at position `at` of a spread or gather launch, in the
+// order that gives each XCD a contiguous run of them: workgroup p goes to XCD p
+// mod 8, and neighbouring bricks, whose halos overlap, then share an L2 (gather
+// of the 64-system set 48.5 -> 43.6 us).
+static void push_bricks(std::vector<WorkItem>& items, int at, int k, int cnt) {
+  constexpr int X = 8;
+  int next[X], lo = 0;
+  for (int r = 0; r < X; r++) {  // run of the positions p = r (mod X) of [at, at + cnt)
+    const int first = (r - at % X + X) % X;
+    next[r] = lo;
+    lo += first < cnt ? (cnt - first + X - 1) / X : 0;
+  }
+  for (int i = 0; i < cnt; i++) items.push_back(WorkItem{k, next[(at + i) % X]++});
+}
+
 void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, const int* orders, int n, int ncu,
                  std::vector<WorkItem>& items, std::vector<Launch>& launches) {
   items.clear();
@@ -266,7 +281,10 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
           lds = fft_cols_lds_bytes(d.bin.nz, d.TXz, d.ax[2].f4 >= 0 ? 1 : 2);
           break;
       }
-      for (int i = 0; i < cnt; i++) items.push_back(WorkItem{k, i});
+      if (stage == BS_SPREAD || stage == BS_GATHER)
+        push_bricks(items, L.count, k, cnt);
+      else
+        for (int i = 0; i < cnt; i++) items.push_back(WorkItem{k, i});
       L.count += cnt;
       L.lds = std::max(L.lds, lds);
     }
@@ -283,15 +301,11 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
   for (int o : {4, 6, 8}) add_stage(BS_GATHER, o, 0, 0);
 }
 
-// Workgroups of a batched launch.  Spread and gather (queue != 0) always run
-// one persistent workgroup per CU (two half-size ones with half_bricks)
-// taking bricks from the launch's work queue (their LDS brick leaves room for
-// no more, and a persistent workgroup saves the start of a new one per brick).  The others
-// run one workgroup per item with wg_per_cu == 0, else wg_per_cu persistent
-// workgroups per CU striding over the items; the plane kernels (cap > 0)
-// cap per CU (one full-size or two half-size workgroups fill a CU).
-static int grid_for(const Tuning& t, int ncu, int count, int cap, bool queue) {
-  if (queue) return std::max(1, std::min(count, ncu * (t.half_bricks ? 2 : 1)));
+// Workgroups of a batched FFT or binning launch: one per item with wg_per_cu ==
+// 0, else wg_per_cu persistent workgroups per CU striding over the items; the
+// plane kernels (cap > 0) cap per CU (one full-size or two half-size
+// workgroups fill a CU).  Spread and gather always run one workgroup per brick.
+static int grid_for(const Tuning& t, int ncu, int count, int cap) {
   if (t.wg_per_cu <= 0) return count;
   const int per_cu = cap > 0 ? cap : t.wg_per_cu;
   return std::max(1, std::min(count, ncu * per_cu));
@@ -304,8 +318,7 @@ static int grid_for(const Tuning& t, int ncu, int count, int cap, bool queue) {
   } while (0)
 
 pme_status enqueue_stages(const std::vector<Launch>& launches, const SysDesc* d_sys, const WorkItem* d_items,
-                          int* d_ctr, const Tuning& t, int ncu, hipStream_t stream, hipEvent_t* tev) {
-  if (launches.size() > (size_t)kMaxLaunches) return set_error(PME_ERR_UNSUPPORTED, "batched solve: too many launches");
+                          const Tuning& t, int ncu, hipStream_t stream, hipEvent_t* tev) {
   // timing slot k: the stages run between events k and k+1
   //   0 bin, 1 spread, 2 x forward and xy-plane forward, 3 y forward, 4 z (+ influence function),
   //   5 y inverse and xy-plane inverse (with the energy/virial reduction), 6 x inverse, 7 gather
@@ -321,13 +334,11 @@ pme_status enqueue_stages(const std::vector<Launch>& launches, const SysDesc* d_
         const Launch& L = launches[li];
         if (L.stage != stage) continue;
         const WorkItem* it = d_items + L.offset;
-        int* ctr = d_ctr + 2 * li;  // this launch's work-queue counters (spread, gather)
-        const bool queue = stage == BS_SPREAD || stage == BS_GATHER;
-        const int grid = grid_for(t, ncu, L.count, stage == BS_PLANE ? (L.half ? 2 : 1) : 0, queue);
+        const int grid = grid_for(t, ncu, L.count, stage == BS_PLANE ? (L.half ? 2 : 1) : 0);
         switch (stage) {
           case BS_BIN: SCHED_HIP(launch_batch_bin(d_sys, it, L.count, grid, L.lds, stream)); break;
           case BS_SPREAD:
-            SCHED_HIP(launch_batch_spread(L.order, t.half_bricks, d_sys, it, L.count, ctr, grid, L.lds, stream));
+            SCHED_HIP(launch_batch_spread(L.order, t.half_bricks, d_sys, it, L.count, L.lds, stream));
             break;
           case BS_FFTX: SCHED_HIP(launch_batch_fft_x(inv ? 1 : 0, d_sys, it, L.count, grid, L.lds, stream)); break;
           case BS_FFTY:
@@ -350,7 +361,7 @@ pme_status enqueue_stages(const std::vector<Launch>& launches, const SysDesc* d_
               SCHED_HIP(launch_batch_cols(2, COL_FWD_SOLVE_INV, 0, L.split, d_sys, it, L.count, grid, L.lds, stream));
             break;
           case BS_GATHER:
-            SCHED_HIP(launch_batch_gather(L.order, t.half_bricks, d_sys, it, L.count, ctr, grid, L.lds, stream));
+            SCHED_HIP(launch_batch_gather(L.order, t.half_bricks, d_sys, it, L.count, L.lds, stream));
             break;
           default: break;
         }

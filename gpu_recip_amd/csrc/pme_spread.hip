@@ -215,33 +215,102 @@ __device__ __forceinline__ void spread_record(const BinArgs& a, float4 p, int x0
   }
 }
 
-// Store phase of a brick: pair i of x-neighbours (lx, lx + 1) of row (ly,
-// lz) converted from fixed point and stored; the second can fall on the
-// row's margin, inside the row's LDS stride, and is then not stored.  WRAP
-// (one brick along x): the high margin is the periodic image of the row
-// start and is added in.  Products of small non-negative integers in 24 bits
-// (edges <= 512), grid offsets in 32 bits (nx*ny < 2^19, offsets < 2^27).
-template <int P, bool WRAP, int NT>
+// A pair of floats (8-byte aligned) stored at agent scope: written through
+// the XCD's L2 at once, instead of left dirty there and written back when the
+// kernel ends.  Only where every brick row is whole 16-byte pieces: 144^3 in
+// rows of 24, order 4, 21.8 -> 19.0 us, 160^3 in rows of 20, order 6, 57.7 -> 56.1
+// us; with other rows the partial pieces of neighbouring bricks meet in memory
+// (150 x 144 x 144 22.2 -> 46 us, 108 x 96 x 96 20.8 -> 30 us).  A batched launch
+// has many bricks per CU and merges the rows of neighbours in the L2 (64-system
+// set: 59.2 us, through 65.7 us).
+__device__ __forceinline__ void store_through(float* g, float a, float b) {
+  const unsigned long long u =
+      (unsigned long long)__float_as_uint(a) | ((unsigned long long)__float_as_uint(b) << 32);
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(g), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Store phase of a brick.  Thread unit = a pair of x-neighbours (lx, lx + 1) of
+// row ly, walking the planes lz = s, s + nseg, ... of its z segment, so the
+// index arithmetic is done once per unit and each pair costs two LDS reads, two
+// conversions and a store.  Even nx: the pairs start at even grid points, so
+// each is one aligned float2 (a brick that starts at an odd one has half a pair
+// at its first point).  A point of a pair can fall on the row's margin, inside
+// the row's LDS stride, and is then not stored.  WRAP (one brick along x): the
+// high margin is the periodic image of the row start and is added in.  Products of
+// small non-negative integers in 24 bits (edges <= 512), grid offsets in 32
+// bits (nx*ny < 2^19, offsets < 2^27).
+// THROUGH: 8-byte aligned pairs go through the L2 (store_through).
+template <int P, bool WRAP, int NT, bool THROUGH>
 __device__ __forceinline__ void store_brick_pairs(const unsigned long long* __restrict__ acc, float* __restrict__ grid,
-                                                  int nx, int ny, int x0, int y0, int z0, int wx, int wy, int hw,
-                                                  int npair, int bxs, int plane) {
+                                                  int nx, int ny, int x0, int y0, int z0, int wx, int wy, int wz,
+                                                  int bxs, int plane) {
+  const bool pairs8 = (nx & 1) == 0;
+  const int odd = pairs8 ? x0 & 1 : 0;
+  const int hw = (wx + odd + 1) >> 1;
+  const int ncol = mul24(hw, wy);
+  const int nseg = max(1, min(sdiv(NT, small_div(ncol)), wz));
   const int nxny = mul24(nx, ny);
-  const SmallDiv dhw = small_div(hw), dwy = small_div(wy);
-  for (int i = threadIdx.x; i < npair; i += NT) {
-    const int t = sdiv(i, dhw);
-    const int lx = 2 * (i - mul24(t, hw));
-    const int lz = sdiv(t, dwy);
-    const int ly = t - mul24(lz, wy);
-    const unsigned long long* row = acc + (mul24(lz, plane) + mul24(ly, bxs) + (P - 1));
-    unsigned long long v0 = row[lx], v1 = row[lx + 1];
-    if (WRAP) {
-      if (lx < P - 1) v0 += row[lx + nx];
-      if (lx + 1 < P - 1) v1 += row[lx + 1 + nx];
+  const SmallDiv dhw = small_div(hw), dcol = small_div(ncol);
+  for (int u = threadIdx.x; u < ncol * nseg; u += NT) {
+    const int s = sdiv(u, dcol);
+    const int c = u - mul24(s, ncol);
+    const int ly = sdiv(c, dhw);
+    const int lx = 2 * (c - mul24(ly, hw)) - odd;
+    const unsigned long long* row = acc + (mul24(s, plane) + mul24(ly, bxs) + (P - 1) + lx);
+    float* g = grid + ((x0 + lx) + mul24(nx, y0 + ly) + mul24(nxny, z0 + s));
+    const bool one = lx >= 0, two = lx + 1 < wx;
+    const int dl = mul24(nseg, plane), dg = mul24(nseg, nxny);
+    for (int lz = s; lz < wz; lz += nseg, row += dl, g += dg) {
+      unsigned long long v0 = row[0], v1 = row[1];
+      if (WRAP) {
+        if (lx < P - 1) v0 += row[nx];
+        if (lx + 1 < P - 1) v1 += row[nx + 1];
+      }
+      const float f0 = from_fixed40(v0), f1 = from_fixed40(v1);
+      if (pairs8 && one && two) {
+        if (THROUGH) store_through(g, f0, f1);
+        else *reinterpret_cast<float2*>(g) = make_float2(f0, f1);
+      } else {
+        if (one) g[0] = f0;
+        if (two) g[1] = f1;
+      }
     }
-    float* g = grid + ((x0 + lx) + mul24(nx, y0 + ly) + mul24(nxny, z0 + lz));
-    g[0] = from_fixed40(v0);
-    if (lx + 1 < wx) g[1] = from_fixed40(v1);
   }
+}
+
+constexpr size_t kNoSlot = (size_t)-1;
+// Orders 6 and 8 only: at 4 a record has too few stencil points for the sort to
+// pay (250k atoms, 144^3: 19.7 against 19.2 us; 64-system set 65.7 against 59.2 us).
+template <int P> constexpr bool kBankOrder = P >= 6;
+
+// Order of a batch of records for the accumulation.  The stencil offsets are
+// the same for every lane, so two lanes of an LDS atomic collide exactly when
+// their stencil bases fall into the same of the 32 eight-byte banks; records in
+// arbitrary order spend more than half of the LDS time on that.  A counting
+// sort by bank (rank within the bank from an LDS counter, a wave-level scan of
+// the 32 counts) and a transposed read, lane j taking the j-th 32nd of the
+// sorted list, spreads the lanes of a wave over the banks.  The list holds
+// record slots.  Integer sums do not depend on the order.
+template <int NT>
+__device__ __forceinline__ size_t bank_order(size_t slot, int bank, bool on, int nbat, int* s_cnt, int* s_list) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  int rank = 0;
+  if (on) rank = atomicAdd(&s_cnt[bank], 1);
+  __syncthreads();
+  const int cnt = s_cnt[lane & 31];
+  int v = cnt;
+#pragma unroll
+  for (int off = 1; off < 32; off <<= 1) {
+    const int t = __shfl_up(v, off, 32);
+    if ((lane & 31) >= off) v += t;
+  }
+  const int start = __shfl(v - cnt, bank, 32);
+  if (on) s_list[start + rank] = (int)slot;
+  __syncthreads();
+  if (tid < 32) s_cnt[tid] = 0;  // for the next batch
+  const int R = (nbat + 31) >> 5;
+  const int at = mul24(tid & 31, R) + (tid >> 5);
+  return (tid >> 5) < R && at < nbat ? (size_t)s_list[at] : kNoSlot;
 }
 
 // Brick b of one grid (one NT-thread workgroup); smem: the workgroup's
@@ -249,10 +318,12 @@ __device__ __forceinline__ void store_brick_pairs(const unsigned long long* __re
 // per batch (an atom whose stencil touches the brick), keeps q*theta_x,
 // theta_y, theta_z in registers and adds its p^3 stencil into the brick
 // (spread_record).
-template <int P, int NT>
+template <int P, int NT, bool THROUGH>
 __device__ __forceinline__ void spread_brick_body(const BinArgs& a, int b, int wxm, int wym, int wzm,
                                                   float* __restrict__ grid, unsigned char* smem) {
   __shared__ int sh_scan[NT / 64];
+  __shared__ int s_cnt[32];
+  __shared__ int s_list[NT];
 
   const int bxs = spread_xstride(wxm, P);
   unsigned long long* acc = reinterpret_cast<unsigned long long*>(smem);
@@ -269,38 +340,57 @@ __device__ __forceinline__ void spread_brick_body(const BinArgs& a, int b, int w
   const int plane = mul24(wym, bxs);
 
   const SegBounds sb = brick_seg_load<false>(a, b);  // in flight while the brick is cleared
-  for (int i = tid; i < acc_n; i += NT) acc[i] = 0ull;
+  for (int i = tid; i < acc_n >> 1; i += NT) reinterpret_cast<ulonglong2*>(acc)[i] = make_ulonglong2(0ull, 0ull);
+  if (tid == 0 && (acc_n & 1)) acc[acc_n - 1] = 0ull;
+  if (tid < 32) s_cnt[tid] = 0;
   const int total = brick_segments<NT>(a, sb, s_pre, s_base, sh_scan);  // ends with a barrier
 
   for (int base = 0; base < total; base += NT) {
-    // records of a batch in a strided order (stride 17, coprime with the
-    // batch size): consecutive records are often atoms of one molecule with
-    // the same stencil rows, and integer sums do not depend on the order
     const int nbat = min(NT, total - base);
-    if (tid >= nbat) break;
-    const int stride = (nbat % 17) ? 17 : ((nbat % 19) ? 19 : 23);
-    const int lt = tid * stride;
-    const int v = base + (lt - mul24(sdiv(lt, small_div(nbat)), nbat));
-    spread_record<P>(a, a.rec_pos[brick_record(a, v, s_pre, s_base)], x0, wx, y0, wy, z0, wz, wrapy, wrapz, bxs,
-                     plane, acc);
+    const bool on = tid < nbat;
+    if (kBankOrder<P>) {
+      size_t slot = on ? brick_record(a, base + tid, s_pre, s_base) : kNoSlot;
+      float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (on) p = a.rec_pos[slot];
+      int ix, iy, iz;
+      float fx, fy, fz;
+      atom_grid_index(a, p, ix, iy, iz, fx, fy, fz);
+      const int dx = local_offset(safe_index(ix, a.nx), x0, wx, a.nx);
+      const int dy = local_offset(safe_index(iy, a.ny), y0, wy, a.ny);
+      const int dz = local_offset(safe_index(iz, a.nz), z0, wz, a.nz);
+      const int bank = (dx + mul24(dy, bxs) + mul24(dz, plane)) & 31;
+      slot = bank_order<NT>(slot, bank, on, nbat, s_cnt, s_list);
+      if (slot != kNoSlot)
+        spread_record<P>(a, a.rec_pos[slot], x0, wx, y0, wy, z0, wz, wrapy, wrapz, bxs, plane, acc);
+      if (base + NT < total) __syncthreads();  // the list and counters are rewritten by the next batch
+    } else {
+      // records of a batch in a strided order (stride 17, coprime with the
+      // batch size): consecutive records are often atoms of one molecule with
+      // the same stencil rows, and integer sums do not depend on the order
+      const int stride = (nbat % 17) ? 17 : ((nbat % 19) ? 19 : 23);
+      const int lt = tid * stride;
+      const int v = base + (lt - mul24(sdiv(lt, small_div(nbat)), nbat));
+      float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (on) p = a.rec_pos[brick_record(a, v, s_pre, s_base)];
+      if (on) spread_record<P>(a, p, x0, wx, y0, wy, z0, wz, wrapy, wrapz, bxs, plane, acc);
+    }
   }
   __syncthreads();
 
-  // the brick is complete: one coalesced store per grid point, no memset
-  // needed; two x-neighbours per thread
-  const int hw = (wx + 1) >> 1;
-  const int npair = hw * wy * wz;
-  if (wrapx)
-    store_brick_pairs<P, true, NT>(acc, grid, a.nx, a.ny, x0, y0, z0, wx, wy, hw, npair, bxs, plane);
+  // the brick is complete: every grid point is stored once, no memset needed
+  if (THROUGH && a.nx % (4 * a.nbx) == 0 && !wrapx)
+    store_brick_pairs<P, false, NT, true>(acc, grid, a.nx, a.ny, x0, y0, z0, wx, wy, wz, bxs, plane);
+  else if (wrapx)
+    store_brick_pairs<P, true, NT, false>(acc, grid, a.nx, a.ny, x0, y0, z0, wx, wy, wz, bxs, plane);
   else
-    store_brick_pairs<P, false, NT>(acc, grid, a.nx, a.ny, x0, y0, z0, wx, wy, hw, npair, bxs, plane);
+    store_brick_pairs<P, false, NT, false>(acc, grid, a.nx, a.ny, x0, y0, z0, wx, wy, wz, bxs, plane);
 }
 
 template <int P>
 __global__ __launch_bounds__(kSpreadBlock) void k_spread_brick(BinArgs a, int wxm, int wym, int wzm,
                                                                float* __restrict__ grid) {
   extern __shared__ __align__(16) unsigned char smem[];
-  spread_brick_body<P, kSpreadBlock>(a, blockIdx.x, wxm, wym, wzm, grid, smem);
+  spread_brick_body<P, kSpreadBlock, true>(a, xcd_brick(blockIdx.x, gridDim.x), wxm, wym, wzm, grid, smem);
 }
 
 size_t spread_lds_bytes(int order, const int wmax[3], int nchunk) {
@@ -327,7 +417,7 @@ hipError_t launch_spread(int order, const BinArgs& a, const int wmax[3], float* 
   return hipGetLastError();
 }
 
-// ---- batched: persistent workgroups over the work items of many systems ----
+// ---- batched: the work items of many systems -----------------------------------
 
 __global__ __launch_bounds__(kBinBlock) void k_batch_bin(const SysDesc* __restrict__ sys,
                                                       const WorkItem* __restrict__ items, int nitems) {
@@ -357,15 +447,11 @@ __global__ __launch_bounds__(kBinBlock) void k_batch_bin(const SysDesc* __restri
 // planned within half the LDS budget (four waves per SIMD: at most 128 VGPRs)
 template <int P, int NT>
 __global__ __launch_bounds__(NT, 4) void k_batch_spread(const SysDesc* __restrict__ sys,
-                                                     const WorkItem* __restrict__ items, int nitems, int* ctr) {
+                                                     const WorkItem* __restrict__ items) {
   extern __shared__ __align__(16) unsigned char smem[];
-  for (int it = blockIdx.x; it < nitems; it = next_item(nitems, ctr)) {
-    const WorkItem w = uniform_item(items[it]);
-    const SysDesc& d = sys[w.sys];
-    spread_brick_body<P, NT>(d.bin, w.idx, d.wmax[0], d.wmax[1], d.wmax[2], d.grid, smem);
-    __syncthreads();
-  }
-  items_done(nitems, ctr);
+  const WorkItem w = uniform_item(items[blockIdx.x]);
+  const SysDesc& d = sys[w.sys];
+  spread_brick_body<P, NT, false>(d.bin, w.idx, d.wmax[0], d.wmax[1], d.wmax[2], d.grid, smem);
 }
 
 hipError_t launch_batch_bin(const SysDesc* sys, const WorkItem* items, int nitems, int grid, size_t lds,
@@ -375,16 +461,15 @@ hipError_t launch_batch_bin(const SysDesc* sys, const WorkItem* items, int nitem
   return hipGetLastError();
 }
 
-hipError_t launch_batch_spread(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems, int* ctr,
-                               int grid, size_t lds, hipStream_t s) {
+hipError_t launch_batch_spread(int order, int half, const SysDesc* sys, const WorkItem* items, int nitems,
+                               size_t lds, hipStream_t s) {
   if (nitems <= 0) return hipSuccess;
   constexpr int H = kSpreadBlock / 2;
 #define PME_BSPREAD(P)                                                                                           \
   if (half)                                                                                                      \
-    hipLaunchKernelGGL((k_batch_spread<P, H>), dim3(grid), dim3(H), lds, s, sys, items, nitems, ctr);            \
+    hipLaunchKernelGGL((k_batch_spread<P, H>), dim3(nitems), dim3(H), lds, s, sys, items);                       \
   else                                                                                                           \
-    hipLaunchKernelGGL((k_batch_spread<P, kSpreadBlock>), dim3(grid), dim3(kSpreadBlock), lds, s, sys, items,    \
-                       nitems, ctr);
+    hipLaunchKernelGGL((k_batch_spread<P, kSpreadBlock>), dim3(nitems), dim3(kSpreadBlock), lds, s, sys, items);
   switch (order) {
     case 4: PME_BSPREAD(4) break;
     case 6: PME_BSPREAD(6) break;
