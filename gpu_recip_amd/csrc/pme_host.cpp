@@ -87,6 +87,7 @@ struct pme_energy_virial_s {
 // yet in the device buffer (it is normally folded into the next kernel);
 // every operation that reads or clears the buffer flushes them first.
 static pme_status flush_pending(pme_recip_t h, hipStream_t target, bool order_target);
+static pme_status ev_copy_out(pme_ev_t ev, hipStream_t target);
 static pme_status ev_flush(pme_ev_t ev, hipStream_t target, bool order_target = true) {
   for (pme_recip_t h : ev->solvers) PME_TRY(flush_pending(h, target, order_target));
   return PME_OK;
@@ -163,9 +164,7 @@ extern "C" pme_status pme_ev_clear_virial(pme_ev_t ev, pme_stream_t stream) {
 
 extern "C" pme_status pme_ev_copy_to_host(pme_ev_t ev, pme_stream_t stream) {
   if (!ev) return fail(PME_ERR_INVALID_ARG, "pme_ev_copy_to_host: null ev");
-  PME_TRY(ev_flush(ev, (hipStream_t)stream));
-  HIP_TRY(hipMemcpyAsync(ev->h_buf, ev->d_buf, kEvBytes, hipMemcpyDeviceToHost, (hipStream_t)stream));
-  return PME_OK;
+  return ev_copy_out(ev, (hipStream_t)stream);
 }
 
 extern "C" pme_status pme_ev_get_energy(pme_ev_t ev, const char* name, double* out) {
@@ -347,6 +346,22 @@ static pme_status flush_pending(pme_recip_t h, hipStream_t target, bool order_ta
     HIP_TRY(hipEventRecord(h->flush_ev, h->stream));
     HIP_TRY(hipStreamWaitEvent(target, h->flush_ev, 0));
   }
+  return PME_OK;
+}
+
+// The buffer to its host mirror.  A reduction pending on the copy's own stream
+// runs in the copy kernel (one solver's; others are flushed first).
+static pme_status ev_copy_out(pme_ev_t ev, hipStream_t target) {
+  pme_recip_t own = nullptr;
+  for (pme_recip_t h : ev->solvers) {
+    if (h->pend_solve == 0 && h->pend_self == 0) continue;
+    if (!own && h->stream == target)
+      own = h;
+    else
+      PME_TRY(flush_pending(h, target, true));
+  }
+  HIP_TRY(launch_copy_out(ev->h_buf, ev->d_buf, kEvBytes, own ? pending_reduce(own) : no_reduce(), target));
+  if (own) own->pend_solve = own->pend_self = 0;
   return PME_OK;
 }
 

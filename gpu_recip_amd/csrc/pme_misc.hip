@@ -24,6 +24,25 @@ hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The energy/virial buffer (2 KB) written to pinned host memory by one
+// workgroup, after a reduction still pending on it: one launch in place of a
+// reduction kernel and a copy command, whose set-up and completion cost more
+// than the bytes (23,559 atoms, 64^3, order 6, self energy, read back every
+// solve: 120 -> 102 us).  red writes into dev, so no restrict here.
+__global__ __launch_bounds__(kBlock) void k_copy_out(unsigned long long* host, const unsigned long long* dev,
+                                                     int nwords, EvReduce red) {
+  ev_reduce_block<kBlock>(red);
+  __syncthreads();  // thread 0's sums, visible to the workgroup
+  for (int k = threadIdx.x; k < nwords; k += kBlock) host[k] = dev[k];
+}
+
+hipError_t launch_copy_out(void* host, const void* dev, size_t bytes, const EvReduce& red, hipStream_t s) {
+  if (bytes % 8) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_copy_out, dim3(1), dim3(kBlock), 0, s, (unsigned long long*)host,
+                     (const unsigned long long*)dev, (int)(bytes / 8), red);
+  return hipGetLastError();
+}
+
 // calc_self_energy_kernel, CudaPMERecip.cu:1252-1275: q*q in FP32, summed in
 // FP64.  Grid-stride with at most 1024 workgroups writing partials; the sum
 // and the -kappa*ccelec/sqrt(pi) factor are applied by ev_reduce_block.
