@@ -4,21 +4,20 @@
 // CudaPMEDirectForce<long long, float> (CudaDirectForce_util.h:184-251,
 // CudaDirectForceKernels.cu:352-400, 506-716).
 //
-// Non-bonded pairs.  The j tiles of the list are split into equal
-// contiguous ranges, one per wave, so the waves carry equal work whatever the
-// spread of the entries' lengths (central-image entries hold tens of tiles,
-// the others a few); a small kernel first maps every j tile to its entry.
-// Each half of a wave walks its half of the range one tile per pass, one j
-// atom per lane, holding the i tile of the tile's entry (32 atoms, moved by
+// Non-bonded pairs.  The waves take the list's j tiles two at a time from a few
+// queues as they finish, so the waves' loads even
+// out whatever the spread of the tiles' pair counts; a small kernel first maps
+// every j tile to its entry.
+// Each half of a wave takes one tile per pass, one j atom per lane, holding the i tile of the tile's entry (32 atoms, moved by
 // the entry's periodic shift on the j side) in LDS and flushing the i-force
 // sums whenever the entry changes.  A pass has two phases.  The check phase
 // tests the 32 x 64 pairs against the cutoff, each lane reading the i atoms
 // at LDS addresses common to its half (broadcast reads) and building a 32-bit
 // mask of its interacting i atoms; the tile's exclusion words, rotated into
 // the same bit order, clear the excluded pairs.  The dense phase packs the
-// wave's interacting pairs into an LDS queue (a wave prefix sum of the mask
-// counts gives each lane its slots) and evaluates them 64 at a time, so the
-// Ewald term runs only for pairs inside the cutoff (about one check in eight
+// wave's interacting pairs into an LDS queue (bit round by bit round, each round a
+// ballot, so that 64 consecutive pairs belong to different j atoms) and evaluates
+// them 64 at a time, so the Ewald term runs only for pairs inside the cutoff (about one check in eight
 // for a 32-atom tile list).  Pair forces are rounded once to 2^40 fixed
 // point and summed with integer LDS atomics per i and per j atom; the sums
 // go to the caller's force array as integer atomics, the j sums after every
@@ -58,15 +57,27 @@ __device__ __forceinline__ float erfc_from_exp(float x, float exp_neg_x2) {
   return acc * t * exp_neg_x2;
 }
 
+// e^{-x} for x >= 0: 2^(-x log2 e) by the hardware exponential (1 ulp) with
+// the product's rounding error and the low part of log2 e carried into a
+// correction factor, so that the result is good to about 1 ulp for every x (the
+// plain product loses x/2 ulp); results below the normal range are 0.
+__device__ __forceinline__ float exp_neg(float x) {
+  const float l2e = 1.44269504f, l2e_lo = 1.92596299e-8f, ln2 = 0.693147181f;
+  const float t = x * l2e;
+  const float lo = fmaf(x, l2e_lo, fmaf(x, l2e, -t));
+  const float y = __builtin_amdgcn_exp2f(-t);
+  return fmaf(y, -lo * ln2, y);
+}
+
 // The EWALD pair term (CudaDirectForceKernels.cu:352-390) for charges already
 // multiplied by ccelec: pot = qq (erfc(kappa r) + fac_m1) / r with fac_m1 = 0
 // for non-bonded pairs, e14fac - 1 for 1-4 interactions and -1 for 1-4
 // exclusions.  Returns fij = (r dU/dr) / r^2, so that fij * (xi - xj) is the
-// gradient on i.  expf is the ROCm device library's.
+// gradient on i.
 __device__ __forceinline__ float ewald_fij(float r2, float rinv, float qq, float fac_m1, const DirectParams& d,
                                            float& pot) {
   const float r = r2 * rinv;
-  const float exp_val = expf(-d.kappa2 * r2);
+  const float exp_val = exp_neg(d.kappa2 * r2);
   const float erfc_val = erfc_from_exp(d.kappa * r, exp_val);
   const float qq_efac_rinv = qq * (erfc_val + fac_m1) * rinv;
   pot = qq_efac_rinv;
@@ -93,25 +104,31 @@ __device__ __forceinline__ unsigned long long pair_fixed(float f) {
   return (unsigned long long)(long long)((double)c * 1099511627776.0);
 }
 
+// The force of a pair and its negative: one range test for the three components,
+// and the negative of the integer where the rounding is to nearest even (which is
+// symmetric).
+__device__ __forceinline__ void pair_fixed3(const float* f, unsigned long long* gi, unsigned long long* gj) {
+  const bool small = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fabsf(f[2])) < 2048.0f;
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    gi[c] = to_fixed_product((double)f[c], 1099511627776.0);
+    gj[c] = 0ull - gi[c];
+  }
+  if (!small) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      gi[c] = pair_fixed(f[c]);
+      gj[c] = pair_fixed(-f[c]);
+    }
+  }
+}
+
 // A pair energy as 2^32 fixed point (integer sums do not depend on which wave
 // takes which pairs); |e| < 2^19 by one FMA, larger ones held inside +-2^30.
 __device__ __forceinline__ long long energy_fixed(float e) {
   if (fabsf(e) < 524288.0f) return (long long)to_fixed_product((double)e, 4294967296.0);
   const float c = fminf(fmaxf(e, -1073741824.0f), 1073741824.0f);
   return (long long)((double)c * 4294967296.0);
-}
-
-// Inclusive prefix sum over the 64 lanes of a wave with DPP moves: shifts by
-// 1, 2, 4 and 8 lanes inside each row of 16, then row 0's and row 2's last
-// lanes into rows 1 and 3, and lane 31 into rows 2 and 3 (all VALU, no LDS).
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-  return v;
 }
 
 // Orders the LDS accesses of the lanes of one wave (all of them issue from
@@ -130,7 +147,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // with integer LDS atomics (exact, so the order does not matter).
 template <int NT>
 __device__ __forceinline__ void write_direct_partial(double elec, double excl, int ish, float sfx, float sfy,
-                                                     float sfz, bool energy, bool virial, double* out) {
+                                                     float sfz, bool energy, bool virial, double* out, size_t st) {
   __shared__ double s_red[2 * (NT / 64)];
   __shared__ unsigned long long s_sf[81];
   const int tid = threadIdx.x;
@@ -148,20 +165,22 @@ __device__ __forceinline__ void write_direct_partial(double elec, double excl, i
     block_sum<2, NT>(v, s_red);
     if (tid == 0) {
       out[0] = v[0];
-      out[1] = v[1];
+      out[st] = v[1];
     }
   }
   if (virial) {
     __syncthreads();
-    for (int k = tid; k < 81; k += NT) out[2 + k] = (double)(long long)s_sf[k] * (1.0 / 1099511627776.0);
+    for (int k = tid; k < 81; k += NT) out[(2 + k) * st] = (double)(long long)s_sf[k] * (1.0 / 1099511627776.0);
   }
 }
 
 // tile_entry[t] = -1 for every tile (the map kernel then fills in the tiles
-// of the entries).
-__global__ __launch_bounds__(256) void k_direct_tile_clear(int n_tile, int* __restrict__ tile_entry) {
+// of the entries), and the chunk queues of the pair kernel to zero.
+__global__ __launch_bounds__(256) void k_direct_tile_clear(int n_tile, int* __restrict__ tile_entry,
+                                                           int* __restrict__ queue) {
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t < n_tile) tile_entry[t] = -1;
+  if (t < kDirQueues) queue[t * kDirQueuePad] = 0;
 }
 
 // Every j tile's entry: tile_entry[t] = e for tileStart <= t <= tileEnd of
@@ -174,6 +193,11 @@ __global__ __launch_bounds__(256) void k_direct_tile_map(int n_ientry, const pme
   const int hi = min(en.tileEnd, n_tile - 1);
   for (int t = max(en.tileStart, 0) + lane; t <= hi; t += 64) tile_entry[t] = e;
 }
+
+// A coordinate, or `far` in place of a NaN or an infinity: the check phase reads
+// the sign of r^2 - roff^2, which a NaN has too; i and j atoms get far values of
+// opposite sign, so no such pair is inside the cutoff.
+__device__ __forceinline__ float far_or(float x, float far) { return fabsf(x) < 1e18f ? x : far; }
 
 // LDS of one wave of the pair kernel
 struct DirWave {
@@ -208,18 +232,22 @@ __device__ __forceinline__ void flush_entry(DirWave& W, int h, int jl, int iatom
   }
 }
 
-// The list's j tiles in chunks of kDirChunk, dealt to the waves in turn
-// (chunk c to wave c mod nwave): every wave sees tiles from the whole list,
-// whose pair density varies tenfold from tile to tile, so the waves' loads
-// even out without a shared counter.  Within a chunk each half of the wave
-// takes kDirChunk / 2 consecutive tiles, one per pass.  The j atoms of a
-// chunk are loaded together at its start, and the tile records (entry, atom
-// index, exclusions) of the wave's next chunk while the current one is
-// processed: one memory round trip per chunk, not a chain of them per pass.
+// The list's j tiles in pairs, one tile per half of a wave and pass.  A wave
+// starts with its own pair of tiles and takes the following ones from a queue:
+// atomics of all XCDs on one address complete about one in 20 ns, so there are
+// kDirQueues of them, each in a cache line of its own, queue q holding the pairs
+// q, q + kDirQueues, ... (every queue sees tiles from the whole list, whose pair
+// density varies tenfold).  The queue runs two pairs ahead: while one is
+// processed, the tile records (entry, atom index, exclusions) of the next are
+// loaded and the ticket of the one after it is under way.  Chunks of 8 tiles
+// dealt to the waves in turn took 91 us for 24,000 atoms (roff 9 A, 33,273 tiles;
+// the mean CU was busy for 57 of them) and 268 us for 96,000; the queue with
+// chunks of 8, 4 and 2 tiles takes 77, 73, 67 and 199, 183, 180 us.
 template <bool ENERGY, bool VIRIAL>
 __global__ __launch_bounds__(kDirWaves * 64) void k_direct_force(DirectParams d, int n_ientry, int n_tile,
                                                                  const pme_ientry* __restrict__ ientry,
                                                                  const int* __restrict__ tile_entry,
+                                                                 int* __restrict__ queue,
                                                                  const int* __restrict__ tile_indj,
                                                                  const pme_tile_excl* __restrict__ tile_excl,
                                                                  const float4* __restrict__ xyzq, int stride,
@@ -238,145 +266,144 @@ __global__ __launch_bounds__(kDirWaves * 64) void k_direct_force(DirectParams d,
     W.fj[c][lane] = 0ull;
   }
   __syncthreads();
-  const int nchunk = (n_tile + kDirChunk - 1) / kDirChunk;
+  const int nchunk = (n_tile + 1) >> 1;  // pairs of tiles
+  // waves and queues (at least one wave per queue)
   const int wtotal = (int)gridDim.x * kDirWaves;
-  int chunk = (int)blockIdx.x * kDirWaves + wv;
+  const int nq = min(kDirQueues, wtotal);
+  const int w0 = (int)blockIdx.x * kDirWaves + wv, q0 = w0 % nq;
+  const int first = q0 + nq * ((wtotal - q0 + nq - 1) / nq);  // first chunk of the queue that no wave starts with
+  int* const ctr = queue + q0 * kDirQueuePad;
+  int chunk = w0;
+  int ticket = 0;  // lane 0
   // the half's current entry
   int cur = -1, cur_lo = 0, cur_hi = -1, cur_ish = 13, cur_i0 = 0;
   float sx = 0.f, sy = 0.f, sz = 0.f;
   long long pot = 0;
-  constexpr int NP = kDirChunk / 2;  // passes per chunk
-  // tile records of the half's NP tiles of a chunk
-  int ne[NP], nindj[NP];
-  unsigned nexcl[NP];
-  auto load_records = [&](int c) {
-#pragma unroll
-    for (int k = 0; k < NP; k++) {
-      const int t = c * kDirChunk + h * NP + k;
-      const bool in = c < nchunk && t < n_tile;
-      ne[k] = in ? tile_entry[t] : -1;
-      nindj[k] = in ? tile_indj[t] : 0;
-      nexcl[k] = in ? tile_excl[t].excl[jl] : 0xffffffffu;
-    }
+  // tile record of the half's tile of a pair
+  int ne = -1, nindj = 0;
+  unsigned nexcl = 0xffffffffu;
+  auto load_record = [&](int c) {
+    const int t = 2 * c + h;
+    const bool in = c < nchunk && t < n_tile;
+    ne = in ? tile_entry[t] : -1;
+    nindj = in ? tile_indj[t] : 0;
+    nexcl = in ? tile_excl[t].excl[jl] : 0xffffffffu;
   };
-  load_records(chunk);
+  auto take = [&]() {
+    if (lane == 0) ticket = atomicAdd(ctr, 1);
+  };
+  take();
+  load_record(chunk);
   while (chunk < nchunk) {
-    const int tbase = chunk * kDirChunk + h * NP;
-    int ce[NP], cindj[NP];
-    unsigned cexcl[NP];
-    float4 cpj[NP];
-#pragma unroll
-    for (int k = 0; k < NP; k++) {
-      ce[k] = ne[k];
-      cindj[k] = nindj[k];
-      cexcl[k] = nexcl[k];
+    const int t = 2 * chunk + h;
+    const int e = ne, indj = nindj;
+    const unsigned excl = nexcl;
+    // the j atoms of this pass, then the record of the next one
+    const float4 pj = e >= 0 ? xyzq[indj + jl] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const int next = first + nq * __builtin_amdgcn_readfirstlane(ticket);
+    if (next < nchunk) take();
+    load_record(next);
+    if (e != cur) {
+      if (cur >= 0) flush_entry<VIRIAL>(W, h, jl, cur_i0, cur_ish, stride, force, s_sf);
+      cur = -1;
+      if (e >= 0 && e < n_ientry) {
+        const pme_ientry en = ientry[e];
+        if (t >= en.tileStart && t <= en.tileEnd) {
+          cur = e;
+          cur_lo = en.tileStart;
+          cur_hi = en.tileEnd;
+          cur_ish = en.ish;
+          cur_i0 = en.iatomStart;
+          box_shift(cur_ish, d, sx, sy, sz);
+          const float4 p = xyzq[cur_i0 + jl];
+          W.xi[h][jl] = make_float4(far_or(p.x, 1e18f), far_or(p.y, 1e18f), far_or(p.z, 1e18f), p.w * (float)kCcelec);
+        }
+      }
     }
-    // the j atoms of this chunk, then the records of the next one
+    wave_lds_sync();
+    const bool ok = cur >= 0 && t >= cur_lo && t <= cur_hi && t < n_tile;
+    // xi - (xj - shift) is the separation of i's image from j
+    const float xjx = far_or(pj.x - sx, -1e18f), xjy = far_or(pj.y - sy, -1e18f), xjz = far_or(pj.z - sz, -1e18f);
+    W.xj[lane] = make_float4(xjx, xjy, xjz, pj.w);
+    // check phase: bit i of m = pair (i, j) inside the cutoff
+    unsigned m = 0u;
 #pragma unroll
-    for (int k = 0; k < NP; k++) cpj[k] = ce[k] >= 0 ? xyzq[cindj[k] + jl] : make_float4(0.f, 0.f, 0.f, 0.f);
-    load_records(chunk + wtotal);
+    for (int g = 3; g >= 0; g--) {
+      float4 pg[8];  // eight i atoms read together, then tested
 #pragma unroll
-    for (int k = 0; k < NP; k++) {
-      const int t = tbase + k;
-      const int e = ce[k];
-      if (e != cur) {
-        if (cur >= 0) flush_entry<VIRIAL>(W, h, jl, cur_i0, cur_ish, stride, force, s_sf);
-        cur = -1;
-        if (e >= 0 && e < n_ientry) {
-          const pme_ientry en = ientry[e];
-          if (t >= en.tileStart && t <= en.tileEnd) {
-            cur = e;
-            cur_lo = en.tileStart;
-            cur_hi = en.tileEnd;
-            cur_ish = en.ish;
-            cur_i0 = en.iatomStart;
-            box_shift(cur_ish, d, sx, sy, sz);
-            const float4 p = xyzq[cur_i0 + jl];
-            W.xi[h][jl] = make_float4(p.x, p.y, p.z, p.w * (float)kCcelec);
-          }
-        }
+      for (int u = 0; u < 8; u++) pg[u] = W.xi[h][8 * g + u];
+#pragma unroll
+      for (int u = 7; u >= 0; u--) {
+        // the sign of r^2 - roff^2, shifted into m
+        const float dx = pg[u].x - xjx, dy = pg[u].y - xjy, dz = pg[u].z - xjz;
+        const float s = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, -d.roff2)));
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(s), 31);
       }
-      wave_lds_sync();
-      const bool ok = cur >= 0 && t >= cur_lo && t <= cur_hi && t < n_tile;
-      const unsigned excl = cexcl[k];
-      const float4 pj = cpj[k];
-      const int indj = cindj[k];
-      // xi - (xj - shift) is the separation of i's image from j
-      const float xjx = pj.x - sx, xjy = pj.y - sy, xjz = pj.z - sz;
-      W.xj[lane] = make_float4(xjx, xjy, xjz, pj.w);
-      // check phase: bit i of m = pair (i, j) inside the cutoff
-      unsigned m = 0u;
-#pragma unroll
-      for (int g = 3; g >= 0; g--) {
-        float4 pg[8];  // eight i atoms read together, then tested
-#pragma unroll
-        for (int u = 0; u < 8; u++) pg[u] = W.xi[h][8 * g + u];
-#pragma unroll
-        for (int u = 7; u >= 0; u--) {
-          const float dx = pg[u].x - xjx, dy = pg[u].y - xjy, dz = pg[u].z - xjz;
-          const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-          m = (m << 1) | (r2 < d.roff2 ? 1u : 0u);
-        }
-      }
-      // bit t of excl[l] excludes i = (l + t) mod 32: rotated left by l it is bit i
-      m &= ~__builtin_amdgcn_alignbit(excl, excl, (32 - jl) & 31);
-      if (!ok) m = 0u;
-      // dense phase: the wave's pairs packed in lane order
-      const int cnt = __popc(m);
-      const int incl = wave_inclusive_scan(cnt);
-      const int total = __builtin_amdgcn_readlane(incl, 63);
-      int slot = incl - cnt;
-      while (m) {
+    }
+    // bit t of excl[l] excludes i = (l + t) mod 32: rotated left by l it is bit i
+    m &= ~__builtin_amdgcn_alignbit(excl, excl, (32 - jl) & 31);
+    if (!ok) m = 0u;
+    // dense phase: the wave's pairs packed round by round, each lane's next
+    // pair per round, so neighbours in the queue have different j atoms
+    int total = 0;
+    for (;;) {
+      const unsigned long long on = __ballot(m != 0u);
+      if (on == 0ull) break;
+      if (m) {
         const int i = __ffs(m) - 1;
         m &= m - 1u;
-        if (slot < 32 * 64) W.pairs[slot] = (unsigned short)(i | (lane << 5));
-        slot++;
+        const int slot = total + __builtin_amdgcn_mbcnt_hi((unsigned)(on >> 32),
+                                                           __builtin_amdgcn_mbcnt_lo((unsigned)on, 0u));
+        W.pairs[slot] = (unsigned short)(i | (lane << 5));  // at most 32 x 64 pairs
       }
-      wave_lds_sync();
-      for (int q = lane; q < total; q += 64) {
-        const unsigned pr = W.pairs[q];
-        const int i = pr & 31, l = pr >> 5, hl = l >> 5;
-        const float4 pi = W.xi[hl][i], pjl = W.xj[l];
-        const float dx = pi.x - pjl.x, dy = pi.y - pjl.y, dz = pi.z - pjl.z;
-        const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-        float pe;
-        const float fij = ewald_fij(r2, rsqrtf(r2), pi.w * pjl.w, 0.0f, d, pe);
-        if (ENERGY) pot += energy_fixed(pe);
-        const float fx = fij * dx, fy = fij * dy, fz = fij * dz;
-        atomicAdd(&W.fi[hl][0][i], pair_fixed(fx));
-        atomicAdd(&W.fi[hl][1][i], pair_fixed(fy));
-        atomicAdd(&W.fi[hl][2][i], pair_fixed(fz));
-        atomicAdd(&W.fj[0][l], pair_fixed(-fx));
-        atomicAdd(&W.fj[1][l], pair_fixed(-fy));
-        atomicAdd(&W.fj[2][l], pair_fixed(-fz));
-      }
-      wave_lds_sync();
-      unsigned long long g[3];
+      total += __popcll(on);
+    }
+    wave_lds_sync();
+    for (int q = lane; q < total; q += 64) {
+      const unsigned pr = W.pairs[q];
+      const int i = pr & 31, l = pr >> 5, hl = l >> 5;
+      const float4 pi = W.xi[hl][i], pjl = W.xj[l];
+      const float dx = pi.x - pjl.x, dy = pi.y - pjl.y, dz = pi.z - pjl.z;
+      const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+      float pe;
+      const float fij = ewald_fij(r2, rsqrtf(r2), pi.w * pjl.w, 0.0f, d, pe);
+      if (ENERGY) pot += energy_fixed(pe);
+      const float f[3] = {fij * dx, fij * dy, fij * dz};
+      unsigned long long gi[3], gj[3];
+      pair_fixed3(f, gi, gj);
 #pragma unroll
       for (int c = 0; c < 3; c++) {
-        g[c] = W.fj[c][lane];
-        W.fj[c][lane] = 0ull;
+        atomicAdd(&W.fi[hl][c][i], gi[c]);
+        atomicAdd(&W.fj[c][l], gj[c]);
       }
-      if (ok && (g[0] | g[1] | g[2])) {
-        atomicAdd(&force[indj + jl], g[0]);
-        atomicAdd(&force[(size_t)(indj + jl) + stride], g[1]);
-        atomicAdd(&force[(size_t)(indj + jl) + 2 * (size_t)stride], g[2]);
-      }
-      wave_lds_sync();
     }
-    chunk += wtotal;
+    wave_lds_sync();
+    unsigned long long g[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      g[c] = W.fj[c][lane];
+      W.fj[c][lane] = 0ull;
+    }
+    if (ok && (g[0] | g[1] | g[2])) {
+      atomicAdd(&force[indj + jl], g[0]);
+      atomicAdd(&force[(size_t)(indj + jl) + stride], g[1]);
+      atomicAdd(&force[(size_t)(indj + jl) + 2 * (size_t)stride], g[2]);
+    }
+    wave_lds_sync();
+    chunk = next;
   }
   if (cur >= 0) flush_entry<VIRIAL>(W, h, jl, cur_i0, cur_ish, stride, force, s_sf);
   if (ENERGY || VIRIAL) {
     if (ENERGY && pot != 0) atomicAdd(&s_pot, (unsigned long long)pot);
     __syncthreads();
-    double* out = partial + (size_t)blockIdx.x * kDirPartial;
+    double* out = partial + blockIdx.x;
+    const size_t st = gridDim.x;
     const int tid = threadIdx.x;
     if (ENERGY && tid == 0) {
       out[0] = (double)(long long)s_pot * (1.0 / 4294967296.0);
-      out[1] = 0.0;
+      out[st] = 0.0;
     }
-    if (VIRIAL && tid < 81) out[2 + tid] = (double)(long long)s_sf[tid] * (1.0 / 1099511627776.0);
+    if (VIRIAL && tid < 81) out[(2 + tid) * st] = (double)(long long)s_sf[tid] * (1.0 / 1099511627776.0);
   }
 }
 
@@ -419,10 +446,10 @@ __global__ __launch_bounds__(kDir14Block) void k_direct_14(DirectParams d, int n
   }
   if (ENERGY || VIRIAL)
     write_direct_partial<kDir14Block>(elec, excl, VIRIAL ? ish_out : -1, sfx, sfy, sfz, ENERGY, VIRIAL,
-                                      partial + (size_t)blockIdx.x * kDirPartial);
+                                      partial + blockIdx.x, gridDim.x);
 }
 
-// Sum the partials of nblk workgroups and add them into the energy/virial
+// Sum the partials of nblk workgroups (slot c of workgroup b at c nblk + b) and add them into the energy/virial
 // buffer: the elec and excl slots and sforce_dp[27][3].  One workgroup per
 // slot; thread k sums workgroups k, k + 256, ... and block_sum adds the
 // threads in fixed order (the same result on every run).
@@ -433,7 +460,7 @@ __global__ __launch_bounds__(256) void k_direct_reduce(const double* __restrict_
   const int c = blockIdx.x;
   if ((c < 2 && !energy) || (c >= 2 && !virial)) return;
   double acc = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += 256) acc += partial[(size_t)b * kDirPartial + c];
+  for (int b = threadIdx.x; b < nblk; b += 256) acc += partial[(size_t)c * nblk + b];
   block_sum<1, 256>(&acc, s_red);
   if (threadIdx.x == 0) {
     if (c == 0) e_elec[0] += acc;
@@ -443,27 +470,28 @@ __global__ __launch_bounds__(256) void k_direct_reduce(const double* __restrict_
 }
 
 hipError_t launch_direct_force(const DirectParams& d, int n_ientry, int n_tile, int nwave,
-                               const pme_ientry* ientry, int* tile_entry, const int* tile_indj,
+                               const pme_ientry* ientry, int* queue, int* tile_entry, const int* tile_indj,
                                const pme_tile_excl* tile_excl, const float4* xyzq, int stride,
                                unsigned long long* force, bool energy, bool virial, double* partial,
                                hipStream_t s) {
   if (n_ientry <= 0 || n_tile <= 0 || nwave <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_direct_tile_clear, dim3((n_tile + 255) / 256), dim3(256), 0, s, n_tile, tile_entry);
+  hipLaunchKernelGGL(k_direct_tile_clear, dim3((n_tile + 255) / 256), dim3(256), 0, s, n_tile, tile_entry, queue);
   hipLaunchKernelGGL(k_direct_tile_map, dim3((n_ientry + 3) / 4), dim3(256), 0, s, n_ientry, ientry, n_tile,
                      tile_entry);
-  const dim3 g(direct_force_blocks(nwave)), b(kDirWaves * 64);
+  const dim3 g(direct_force_blocks(nwave));
+  const dim3 b(kDirWaves * 64);
   if (energy && virial)
-    hipLaunchKernelGGL((k_direct_force<true, true>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, tile_indj,
-                       tile_excl, xyzq, stride, force, partial);
+    hipLaunchKernelGGL((k_direct_force<true, true>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, queue,
+                       tile_indj, tile_excl, xyzq, stride, force, partial);
   else if (energy)
-    hipLaunchKernelGGL((k_direct_force<true, false>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, tile_indj,
-                       tile_excl, xyzq, stride, force, partial);
+    hipLaunchKernelGGL((k_direct_force<true, false>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, queue,
+                       tile_indj, tile_excl, xyzq, stride, force, partial);
   else if (virial)
-    hipLaunchKernelGGL((k_direct_force<false, true>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, tile_indj,
-                       tile_excl, xyzq, stride, force, partial);
+    hipLaunchKernelGGL((k_direct_force<false, true>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, queue,
+                       tile_indj, tile_excl, xyzq, stride, force, partial);
   else
-    hipLaunchKernelGGL((k_direct_force<false, false>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, tile_indj,
-                       tile_excl, xyzq, stride, force, partial);
+    hipLaunchKernelGGL((k_direct_force<false, false>), g, b, 0, s, d, n_ientry, n_tile, ientry, tile_entry, queue,
+                       tile_indj, tile_excl, xyzq, stride, force, partial);
   return hipGetLastError();
 }
 
@@ -496,8 +524,8 @@ hipError_t launch_direct_reduce(const double* partial, int nblk, bool energy, bo
 int direct_force_blocks(int nwave) { return (nwave + kDirWaves - 1) / kDirWaves; }
 
 int direct_force_waves(int n_tile, int ncu) {
-  // 16 waves per CU (four workgroups of kDirWaves), at most one per chunk
-  return std::max(1, std::min(ncu * 16, (n_tile + kDirChunk - 1) / kDirChunk));
+  // 16 waves per CU (four workgroups of kDirWaves), at most one per pair of tiles
+  return std::max(1, std::min(ncu * 16, (n_tile + 1) / 2));
 }
 int direct_14_blocks(int n) { return (n + kDir14Block - 1) / kDir14Block; }
 

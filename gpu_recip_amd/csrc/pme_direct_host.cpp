@@ -46,7 +46,7 @@ struct pme_direct_s {
   int in14_cap = 0, ex14_cap = 0;
   double* partial = nullptr;    // [partial_cap * kDirPartial] per-workgroup partials
   int partial_cap = 0;
-  int* tile_entry = nullptr;    // [tile_cap] entry of every j tile of the list
+  int* tile_entry = nullptr;    // chunk queues [kDirQueueInts], then [tile_cap] entry of every j tile of the list
   int tile_cap = 0;
   int ncu = 0;                  // compute units of the device
 };
@@ -244,10 +244,11 @@ extern "C" pme_status pme_direct_calc_force(pme_direct_t h, const void* d_xyzq, 
     (void)hipFree(h->tile_entry);
     h->tile_entry = nullptr;
     h->tile_cap = 0;
-    HIP_TRY(hipMalloc(&h->tile_entry, sizeof(int) * (size_t)nlist->n_tile));
+    HIP_TRY(hipMalloc(&h->tile_entry, sizeof(int) * (kDirQueueInts + (size_t)nlist->n_tile)));
     h->tile_cap = nlist->n_tile;
   }
   HIP_TRY(launch_direct_force(h->d, nlist->n_ientry, nlist->n_tile, nwave, nlist->ientry, h->tile_entry,
+                              h->tile_entry + kDirQueueInts,
                               nlist->tile_indj, nlist->tile_excl, (const float4*)d_xyzq, stride,
                               reinterpret_cast<unsigned long long*>(d_force), ce, cv, h->partial, s));
   HIP_TRY(launch_direct_reduce(h->partial, nblk, ce, cv, h->e_elec, h->e_excl, h->sforce_dp, s));

@@ -416,11 +416,13 @@ struct DirectParams {
   float e14fac;
 };
 constexpr int kDirWaves = 4;         // waves per non-bonded workgroup
-constexpr int kDirChunk = 8;         // j tiles per chunk of the pair kernel (kDirChunk / 2 per half-wave)
+constexpr int kDirQueues = 16;       // chunk queues of the pair kernel
+constexpr int kDirQueuePad = 32;     // ints per queue (a cache line)
+constexpr int kDirQueueInts = kDirQueues * kDirQueuePad;
 constexpr int kDir14Block = 256;     // 1-4 entries per workgroup
 constexpr int kDirPartial = 2 + 81;  // doubles per workgroup partial: elec, excl, sforce[27][3]
 hipError_t launch_direct_force(const DirectParams& d, int n_ientry, int n_tile, int nwave,
-                               const pme_ientry* ientry, int* tile_entry, const int* tile_indj,
+                               const pme_ientry* ientry, int* queue, int* tile_entry, const int* tile_indj,
                                const pme_tile_excl* tile_excl, const float4* xyzq, int stride,
                                unsigned long long* force, bool energy, bool virial, double* partial,
                                hipStream_t s);
