@@ -14,6 +14,7 @@
 // reference's r2c z-stage + scalar_sum + c2r z-stage in one read and one write
 // of the spectrum.
 #include "pme_internal.hpp"
+#include "pme_zpass.hpp"
 
 namespace pme {
 
@@ -512,436 +513,6 @@ hipError_t launch_fft_plane_inv(const float2* cg, float* grid, int nx, int ny, i
   return hipGetLastError();
 }
 
-// ------------------------------------------------------- influence function --
-
-// eterm at (k1, k2, k3) and the energy/virial terms of that point,
-// scalar_sum_ortho_kernel CudaPMERecip.cu:671-704
-__device__ __forceinline__ float eterm_at(const SolveArgs& s, int k1, int k2, int k3, float& mh1, float& mh2,
-                                          float& mh3, float& msq_inv) {
-  const int m1 = k1 >= s.nf1 ? k1 - s.n1 : k1;
-  const int m2 = k2 >= s.nf2 ? k2 - s.n2 : k2;
-  const int m3 = k3 >= s.nf3 ? k3 - s.n3 : k3;
-  mh1 = s.r1 * (float)m1;
-  mh2 = s.r2 * (float)m2;
-  mh3 = s.r3 * (float)m3;
-  // grouped as in solve_lines, which takes the (k1, k2) factors out of its
-  // loop over k3, so both give the same value; the fused multiply-adds are
-  // explicit so that every kernel rounds them alike
-  const float s12 = fmaf(mh2, mh2, mh1 * mh1);
-  const float msq = fmaf(mh3, mh3, s12);
-  const float p12 = s.piv_inv * s.pf1[k1] * s.pf2[k2];
-  // hardware reciprocal and exponential (1-2 ulp), as the reference's fast-math build
-  msq_inv = __builtin_amdgcn_rcpf(msq);
-  return __expf(-s.fac * msq) * p12 * s.pf3[k3] * msq_inv;
-}
-
-// Multiply one half-spectrum point by eterm; accumulate energy/virial with
-// the reference's weights (mirror term for every k1 >= 1, :708-741).  The
-// mirror point (n1-k1, -k2, -k3) has the same |m|^2 and, bsp_mod being
-// symmetric, the same eterm; its m components are -m except on a Nyquist
-// plane of an even axis (m = -n/2 maps to itself), so the diagonal terms
-// double and each off-diagonal term m_a m_b doubles or cancels.
-__device__ __forceinline__ float2 solve_point(const SolveArgs& s, float2 q, int k1, int k2, int k3, double* acc) {
-  if ((k1 | k2 | k3) == 0) return make_float2(0.f, 0.f);
-  float mh1, mh2, mh3, msq_inv;
-  const float eterm = eterm_at(s, k1, k2, k3, mh1, mh2, mh3, msq_inv);
-  if (s.calc_ev) {
-    const float q2 = fmaf(q.y, q.y, q.x * q.x);
-    const float tmp1 = eterm * q2;
-    const float vterm = 2.0f * (s.fac + msq_inv);
-    const float tmp2 = tmp1 * vterm;
-    // weight of the point (1) plus its mirror (1 when k1 >= 1)
-    const double w = k1 >= 1 ? 2.0 : 1.0;
-    // mirror sign of each m component: +1 when it maps to itself
-    const bool f1 = !(2 * k1 == s.n1), f2 = !(2 * k2 == s.n2 || k2 == 0), f3 = !(2 * k3 == s.n3 || k3 == 0);
-    const double w12 = k1 >= 1 ? (f1 == f2 ? 2.0 : 0.0) : 1.0;
-    const double w13 = k1 >= 1 ? (f1 == f3 ? 2.0 : 0.0) : 1.0;
-    const double w23 = k1 >= 1 ? (f2 == f3 ? 2.0 : 0.0) : 1.0;
-    acc[0] += w * (double)tmp1;
-    acc[1] += w * (double)(tmp1 * (vterm * mh1 * mh1 - 1.0f));
-    acc[2] += w12 * (double)(tmp2 * mh1 * mh2);
-    acc[3] += w13 * (double)(tmp2 * mh1 * mh3);
-    acc[4] += w * (double)(tmp1 * (vterm * mh2 * mh2 - 1.0f));
-    acc[5] += w23 * (double)(tmp2 * mh2 * mh3);
-    acc[6] += w * (double)(tmp1 * (vterm * mh3 * mh3 - 1.0f));
-  }
-  return cscale(q, eterm);
-}
-
-// eterm of a triclinic box at mapped wave numbers (m1, m2, m3), k3 = its z
-// index: m-hat = m1 R[0][:] + m2 R[1][:] + m3 R[2][:] (rows of recip).
-__device__ __forceinline__ float eterm_tric(const SolveArgs& s, int k1, int k2, int k3, int m1, int m2, int m3,
-                                            float* mh, float& msq_inv) {
-  const float f1 = (float)m1, f2 = (float)m2, f3 = (float)m3;
-  mh[0] = fmaf(s.rt[6], f3, fmaf(s.rt[3], f2, s.rt[0] * f1));
-  mh[1] = fmaf(s.rt[7], f3, fmaf(s.rt[4], f2, s.rt[1] * f1));
-  mh[2] = fmaf(s.rt[8], f3, fmaf(s.rt[5], f2, s.rt[2] * f1));
-  const float msq = fmaf(mh[2], mh[2], fmaf(mh[1], mh[1], mh[0] * mh[0]));
-  msq_inv = __builtin_amdgcn_rcpf(msq);
-  return __expf(-s.fac * msq) * (s.piv_inv * s.pf1[k1] * s.pf2[k2]) * s.pf3[k3] * msq_inv;
-}
-
-// energy and virial terms of one point (weight 1), the order of acc as in solve_point
-__device__ __forceinline__ void ev_terms(const SolveArgs& s, float eterm, float q2, const float* mh, float msq_inv,
-                                         double* acc) {
-  const float tmp1 = eterm * q2;
-  const float vterm = 2.0f * (s.fac + msq_inv);
-  const float tmp2 = tmp1 * vterm;
-  acc[0] += (double)tmp1;
-  acc[1] += (double)(tmp1 * (vterm * mh[0] * mh[0] - 1.0f));
-  acc[2] += (double)(tmp2 * mh[0] * mh[1]);
-  acc[3] += (double)(tmp2 * mh[0] * mh[2]);
-  acc[4] += (double)(tmp1 * (vterm * mh[1] * mh[1] - 1.0f));
-  acc[5] += (double)(tmp2 * mh[1] * mh[2]);
-  acc[6] += (double)(tmp1 * (vterm * mh[2] * mh[2] - 1.0f));
-}
-
-// solve_point for a triclinic box: the same weights (the point, plus its
-// mirror (n1-k1, -k2, -k3) for every k1 >= 1), but the mirror's m-hat is not
-// minus the point's on a Nyquist plane, so its eterm and virial terms are
-// evaluated from its own wave numbers.
-__device__ __forceinline__ float2 solve_point_tric(const SolveArgs& s, float2 q, int k1, int k2, int k3, double* acc) {
-  if ((k1 | k2 | k3) == 0) return make_float2(0.f, 0.f);
-  const int m1 = k1 >= s.nf1 ? k1 - s.n1 : k1;
-  const int m2 = k2 >= s.nf2 ? k2 - s.n2 : k2;
-  const int m3 = k3 >= s.nf3 ? k3 - s.n3 : k3;
-  float mh[3], msq_inv;
-  const float eterm = eterm_tric(s, k1, k2, k3, m1, m2, m3, mh, msq_inv);
-  if (s.calc_ev) {
-    const float q2 = fmaf(q.y, q.y, q.x * q.x);
-    ev_terms(s, eterm, q2, mh, msq_inv, acc);
-    if (k1 >= 1) {
-      const int k1s = s.n1 - k1, k2s = k2 ? s.n2 - k2 : 0, k3s = k3 ? s.n3 - k3 : 0;
-      const int m1s = k1s >= s.nf1 ? k1s - s.n1 : k1s;
-      const int m2s = k2s >= s.nf2 ? k2s - s.n2 : k2s;
-      const int m3s = k3s >= s.nf3 ? k3s - s.n3 : k3s;
-      float ms[3], msq_inv_s;
-      const float eterm_s = eterm_tric(s, k1s, k2s, k3s, m1s, m2s, m3s, ms, msq_inv_s);
-      ev_terms(s, eterm_s, q2, ms, msq_inv_s, acc);
-    }
-  }
-  return cscale(q, eterm);
-}
-
-// The influence function over the z lines of a column tile (in LDS, point j
-// of line l at res[j * TX + l]; lines l < nl are kx = kx0 + l at ky = k2).
-// Thread t owns line t mod TX and visits k3 = t / TX, t / TX + kBlock / TX,
-// ..., so the (k1, k2) factors of eterm and of the energy/virial terms are
-// formed once per thread: scalar_sum_ortho_kernel CudaPMERecip.cu:671-747
-// per point, with the sums over k3 of one line taken before the line's
-// constant factors are applied.  Per line, with the point weight w (2 when
-// k1 >= 1: the point and its mirror), tmp1 = eterm |Q|^2, tmp2 = tmp1 vterm:
-//   E   += w sum tmp1                  V11 += w (mh1^2 sum tmp2 - sum tmp1)
-//   V22 += w (mh2^2 sum tmp2 - sum tmp1)  V33 += w (sum tmp2 mh3^2 - sum tmp1)
-//   V12 += w12 mh1 mh2 sum tmp2      V13 += mh1 sum w13 tmp2 mh3
-//   V23 += mh2 sum w23 tmp2 mh3
-// (the off-diagonal mirror weights are those of solve_point; w13 and w23
-// depend on k3 through the zero/Nyquist test of m3).
-__device__ __forceinline__ void solve_lines(const SolveArgs& s, float2* __restrict__ res, int n, int TX, int nl,
-                                            int c0, int hxd, double* acc) {
-  const int tid = threadIdx.x;
-  const SmallDiv dtx = small_div(TX);
-  const int j0 = sdiv(tid, dtx);
-  const int l = tid - j0 * TX;
-  const int jstep = sdiv(kBlock, dtx);  // >= 4: column tiles are at most 64 wide
-  static_assert(kBlock >= 4 * 64, "solve_lines: every line needs a thread");
-  if (j0 >= jstep || l >= nl) return;
-  // line c0 + l of the z pass: flattened (ky, kx) of the z plane, rows of hxd
-  const int c = c0 + l;
-  const int k2 = sdiv(c, small_div(hxd));
-  const int k1 = c - k2 * hxd;
-  const int m1 = k1 >= s.nf1 ? k1 - s.n1 : k1;
-  const int m2 = k2 >= s.nf2 ? k2 - s.n2 : k2;
-  const float mh1 = s.r1 * (float)m1;
-  const float mh2 = s.r2 * (float)m2;
-  const float s12 = fmaf(mh2, mh2, mh1 * mh1);
-  const float p12 = s.piv_inv * s.pf1[k1] * s.pf2[k2];
-  const bool f1 = !(2 * k1 == s.n1), f2 = !(2 * k2 == s.n2 || k2 == 0);
-  const bool k1pos = k1 >= 1;
-  double sA = 0.0, sB = 0.0, sC = 0.0, sD13 = 0.0, sD23 = 0.0;
-  for (int j = j0; j < n; j += jstep) {
-    float2* pt = res + mul24(j, TX) + l;
-    if ((k1 | k2 | j) == 0) {
-      *pt = make_float2(0.f, 0.f);
-      continue;
-    }
-    const int m3 = j >= s.nf3 ? j - s.n3 : j;
-    const float mh3 = s.r3 * (float)m3;
-    const float msq = fmaf(mh3, mh3, s12);
-    const float msq_inv = __builtin_amdgcn_rcpf(msq);
-    const float eterm = __expf(-s.fac * msq) * p12 * s.pf3[j] * msq_inv;
-    const float2 q = *pt;
-    if (s.calc_ev) {
-      const float q2 = fmaf(q.y, q.y, q.x * q.x);
-      const float tmp1 = eterm * q2;
-      const float vterm = 2.0f * (s.fac + msq_inv);
-      const float tmp2 = tmp1 * vterm;
-      const float t3 = tmp2 * mh3;
-      const bool f3 = !(2 * j == s.n3 || j == 0);
-      const float w13 = k1pos ? (f1 == f3 ? 2.f : 0.f) : 1.f;
-      const float w23 = k1pos ? (f2 == f3 ? 2.f : 0.f) : 1.f;
-      sA += (double)tmp1;
-      sB += (double)tmp2;
-      sC += (double)(t3 * mh3);
-      sD13 += (double)(w13 * t3);
-      sD23 += (double)(w23 * t3);
-    }
-    *pt = cscale(q, eterm);
-  }
-  if (s.calc_ev) {
-    const double w = k1pos ? 2.0 : 1.0;
-    const double w12 = k1pos ? (f1 == f2 ? 2.0 : 0.0) : 1.0;
-    const double a1 = (double)mh1, a2 = (double)mh2;
-    acc[0] += w * sA;
-    acc[1] += w * (a1 * a1 * sB - sA);
-    acc[2] += w12 * a1 * a2 * sB;
-    acc[3] += a1 * sD13;
-    acc[4] += w * (a2 * a2 * sB - sA);
-    acc[5] += a2 * sD23;
-    acc[6] += w * (sC - sA);
-  }
-}
-
-// Per-workgroup energy/virial partial (fixed summation order inside the
-// workgroup).  The total is formed later by ev_reduce_block in one workgroup.
-__device__ __forceinline__ void ev_partial(const SolveArgs& s, double* acc, double* sh, int blk) {
-  block_sum<7>(acc, sh);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int c = 0; c < 7; c++) s.partial[(size_t)blk * 7 + c] = acc[c];
-  }
-}
-
-// ---- z pass as a register four-step FFT -------------------------------------
-// n = N1 N2, j = j2 + N2 j1, k = k1 + N1 k2:
-//   X[k1 + N1 k2] = sum_j2 w_N2^{j2 k2} w_n^{j2 k1} sum_j1 w_N1^{j1 k1} x[j2 + N2 j1].
-// Work unit (line l, q): in the forward half q = j2 (an N1-point DFT of the
-// column j2 + N2 j1 in registers, the twiddle w_n^{j2 k1}, one LDS
-// exchange), then q = k1 (an N2-point DFT in registers).  That thread then
-// holds the whole line's spectrum at k3 = k1 + N1 k2, applies the influence
-// function there and runs the inverse the same way back (the conjugate
-// steps in reverse order).  Two LDS exchanges per direction instead of one
-// per radix stage, and no index arithmetic inside the DFTs.
-#define PME_F4_PAIRS(X)                                                                             \
-  X(0, 4, 4) X(1, 4, 5) X(2, 4, 6) X(3, 5, 5) X(4, 3, 9) X(5, 5, 6) X(6, 4, 8) X(7, 6, 6) X(8, 5, 8) \
-  X(9, 5, 9) X(10, 6, 8) X(11, 5, 10) X(12, 6, 9) X(13, 6, 10) X(14, 8, 8) X(15, 8, 9) X(16, 5, 15)  \
-  X(17, 8, 10) X(18, 9, 9) X(19, 9, 10) X(20, 8, 12) X(21, 10, 10) X(22, 9, 12) X(23, 10, 12)        \
-  X(24, 8, 16) X(25, 9, 15) X(26, 12, 12) X(27, 10, 15) X(28, 10, 16) X(29, 12, 15) X(30, 12, 16)
-
-int four_step_code(int n) {
-#define PME_F4_CODE(c, a, b) \
-  if (n == (a) * (b)) return c;
-  PME_F4_PAIRS(PME_F4_CODE)
-#undef PME_F4_CODE
-  return -1;
-}
-
-// Register class of a factor pair.  A kernel that dispatches over several
-// pairs is allocated the registers of their union, which grows well beyond
-// the largest single pair (all 31 pairs and the Stockham stages: 157 VGPRs,
-// three waves per SIMD; one pair: 72 to 118).  The batched z pass therefore
-// has one kernel per class: class 0 holds the pairs with N2 <= 10 and 5 x 15
-// (75, a common edge; held to 128 VGPRs, four waves per SIMD, with three
-// spilled), class 1 the rest (125 VGPRs).
-constexpr int f4_class_of(int n1, int n2) { return (n2 <= 10 || (n1 == 5 && n2 == 15)) ? 0 : 1; }
-int four_step_code_for_plan(const RadixPlan& rp) {
-  const int code = four_step_code(rp.n);
-  int a = 0, b = 0;
-  return (rp.f4a > 0 && code >= 0 && four_step_pair(code, &a, &b) && a == rp.f4a && b == rp.f4b) ? code : -1;
-}
-
-bool four_step_pair(int code, int* n1, int* n2) {
-#define PME_F4_PAIR(c, a, b) \
-  if (code == (c)) {         \
-    *n1 = (a);               \
-    *n2 = (b);               \
-    return true;             \
-  }
-  PME_F4_PAIRS(PME_F4_PAIR)
-#undef PME_F4_PAIR
-  return false;
-}
-
-int four_step_class(int code) {
-#define PME_F4_CLS(c, a, b) \
-  if (code == (c)) return f4_class_of(a, b);
-  PME_F4_PAIRS(PME_F4_CLS)
-#undef PME_F4_CLS
-  return -1;
-}
-
-// eterm of one point of a z line; (k1, k2) factors precomputed (as in
-// solve_lines, so the value is the same)
-struct LineFactors {
-  float mh1, mh2, s12, p12;
-  bool f1, f2, k1pos;
-  int k1, k2;
-};
-__device__ __forceinline__ LineFactors line_factors(const SolveArgs& s, int k1, int k2) {
-  LineFactors f;
-  const int m1 = k1 >= s.nf1 ? k1 - s.n1 : k1;
-  const int m2 = k2 >= s.nf2 ? k2 - s.n2 : k2;
-  f.mh1 = s.r1 * (float)m1;
-  f.mh2 = s.r2 * (float)m2;
-  f.s12 = fmaf(f.mh2, f.mh2, f.mh1 * f.mh1);
-  f.p12 = s.piv_inv * s.pf1[k1] * s.pf2[k2];
-  f.f1 = !(2 * k1 == s.n1);
-  f.f2 = !(2 * k2 == s.n2 || k2 == 0);
-  f.k1pos = k1 >= 1;
-  f.k1 = k1;
-  f.k2 = k2;
-  return f;
-}
-
-// Q <- eterm Q at k3 of the line; energy/virial sums as in solve_lines
-__device__ __forceinline__ float2 solve_line_point(const SolveArgs& s, const LineFactors& f, int k3, float2 q,
-                                                   double* sums) {
-  if ((f.k1 | f.k2 | k3) == 0) return make_float2(0.f, 0.f);
-  const int m3 = k3 >= s.nf3 ? k3 - s.n3 : k3;
-  const float mh3 = s.r3 * (float)m3;
-  const float msq = fmaf(mh3, mh3, f.s12);
-  const float msq_inv = __builtin_amdgcn_rcpf(msq);
-  const float eterm = __expf(-s.fac * msq) * f.p12 * s.pf3[k3] * msq_inv;
-  if (s.calc_ev) {
-    const float q2 = fmaf(q.y, q.y, q.x * q.x);
-    const float tmp1 = eterm * q2;
-    const float vterm = 2.0f * (s.fac + msq_inv);
-    const float tmp2 = tmp1 * vterm;
-    const float t3 = tmp2 * mh3;
-    const bool f3 = !(2 * k3 == s.n3 || k3 == 0);
-    const float w13 = f.k1pos ? (f.f1 == f3 ? 2.f : 0.f) : 1.f;
-    const float w23 = f.k1pos ? (f.f2 == f3 ? 2.f : 0.f) : 1.f;
-    sums[0] += (double)tmp1;
-    sums[1] += (double)tmp2;
-    sums[2] += (double)(t3 * mh3);
-    sums[3] += (double)(w13 * t3);
-    sums[4] += (double)(w23 * t3);
-  }
-  return cscale(q, eterm);
-}
-
-__device__ __forceinline__ void fold_line_sums(const LineFactors& f, const double* sums, double* acc) {
-  const double w = f.k1pos ? 2.0 : 1.0;
-  const double w12 = f.k1pos ? (f.f1 == f.f2 ? 2.0 : 0.0) : 1.0;
-  const double a1 = (double)f.mh1, a2 = (double)f.mh2;
-  acc[0] += w * sums[0];
-  acc[1] += w * (a1 * a1 * sums[1] - sums[0]);
-  acc[2] += w12 * a1 * a2 * sums[1];
-  acc[3] += a1 * sums[3];
-  acc[4] += w * (a2 * a2 * sums[1] - sums[0]);
-  acc[5] += a2 * sums[4];
-  acc[6] += w * (sums[2] - sums[0]);
-}
-
-// One column tile of the z pass (as fft_cols_body<COL_FWD_SOLVE_INV>) with
-// n = N1 N2: TX consecutive lines c0 .. c0+TX-1 of the flattened (ky, kx)
-// index of a z plane (rows of hxd), point j of line l at base + j pt_stride
-// + l.  sm: twiddles (ntw) and ONE n*TX buffer b: the first half reads its
-// columns straight from HBM into registers and writes b at (k1 N2 + j2); the
-// middle pass reads and rewrites the same N2 points of b per unit (in place);
-// the last half reads b and stores straight to HBM.  Lanes run along l, so
-// every HBM access of a wave is two runs of TX consecutive float2.
-template <int N1, int N2>
-__device__ __forceinline__ void zsolve_four_step(float2* __restrict__ cg, int hx, int TX, long long pt_stride,
-                                                 long long outer_stride, const AxisArgs& ax, const SolveArgs& sa,
-                                                 int tx, int ty, int blk, float2* sm, int hxd) {
-  __shared__ double sh_red[7 * (kBlock / 64)];
-  const int tid = threadIdx.x;
-  float2* tw = sm;
-  float2* b = sm + ax.ntw;
-  for (int i = tid; i < ax.ntw; i += kBlock) tw[i] = ax.tw[i];
-  const int ts = ax.rp.tstride;
-  const int kx0 = tx * TX;
-  const int nl = min(TX, hx - kx0);
-  // the tile's first point (uniform) and 32-bit point offsets from it: a z
-  // line spans n * pt_stride < 2^27 points (edges <= 512)
-  float2* __restrict__ tile = cg + ((size_t)kx0 + (size_t)ty * (size_t)outer_stride);
-  const unsigned pst = (unsigned)pt_stride;
-  const int tsh = __builtin_ctz(TX);  // TX is a power of two (pick_fft_tiles)
-  // forward, first half: unit (l, j2), column j2 + N2 j1 loaded from HBM
-  for (int u0 = 0; u0 < N2 * TX; u0 += kBlock) {
-    const int u = u0 + tid;
-    const int j2 = (u >> tsh);
-    const int l = u - j2 * TX;
-    const bool live = u < N2 * TX;
-    float2 x[N1];
-    const unsigned o = (unsigned)j2 * pst + (unsigned)l;
-#pragma unroll
-    for (int j1 = 0; j1 < N1; j1++)
-      x[j1] = (live && l < nl) ? tile[o + (unsigned)(N2 * j1) * pst] : make_float2(0.f, 0.f);
-    if (u0 == 0) __syncthreads();  // twiddles in LDS (uniform branch)
-    if (live) {
-      DftN<N1, -1>::run(x);
-#pragma unroll
-      for (int k1 = 0; k1 < N1; k1++) {
-        const float2 y = k1 == 0 ? x[0] : cmul(x[k1], tw[mul24(j2 * k1, ts)]);
-        b[(k1 * N2 + j2) * TX + l] = y;
-      }
-    }
-  }
-  __syncthreads();
-  // forward second half, influence function, inverse first half: unit (l, k1),
-  // in place on the N2 points (k1 N2 + j2) of b
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int u = tid; u < N1 * TX; u += kBlock) {
-    const int k1 = (u >> tsh);
-    const int l = u - k1 * TX;
-    float2 X[N2];
-#pragma unroll
-    for (int j2 = 0; j2 < N2; j2++) X[j2] = b[(k1 * N2 + j2) * TX + l];
-    DftN<N2, -1>::run(X);  // X[k2]: point k3 = k1 + N1 k2
-    if (l < nl) {
-      const int ky = sdiv(kx0 + l, small_div(hxd));
-      const LineFactors f = line_factors(sa, kx0 + l - ky * hxd, ky);
-      double sums[5] = {0, 0, 0, 0, 0};
-#pragma unroll
-      for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_point(sa, f, k1 + N1 * k2, X[k2], sums);
-      if (sa.calc_ev) fold_line_sums(f, sums, acc);
-    }
-    DftN<N2, +1>::run(X);  // X[j2]
-#pragma unroll
-    for (int j2 = 0; j2 < N2; j2++) {
-      const float2 t = tw[mul24(j2 * k1, ts)];
-      const float2 z = j2 == 0 ? X[0] : cmul(X[j2], make_float2(t.x, -t.y));
-      b[(k1 * N2 + j2) * TX + l] = z;
-    }
-  }
-  __syncthreads();
-  // inverse second half: unit (l, j2), stored straight to HBM
-  for (int u = tid; u < N2 * TX; u += kBlock) {
-    const int j2 = (u >> tsh);
-    const int l = u - j2 * TX;
-    float2 z[N1];
-#pragma unroll
-    for (int k1 = 0; k1 < N1; k1++) z[k1] = b[(k1 * N2 + j2) * TX + l];
-    DftN<N1, +1>::run(z);  // z[j1]: point j = j2 + N2 j1
-    if (l < nl) {
-      const unsigned o = (unsigned)j2 * pst + (unsigned)l;
-#pragma unroll
-      for (int j1 = 0; j1 < N1; j1++) tile[o + (unsigned)(N2 * j1) * pst] = z[j1];
-    }
-  }
-  if (sa.calc_ev) ev_partial(sa, acc, sh_red, blk);
-}
-
-// the pairs of register class CLS only
-template <int CLS>
-__device__ __forceinline__ void zsolve_four_step_dispatch(int code, float2* __restrict__ cg, int hx, int TX,
-                                                          long long pt_stride, long long outer_stride,
-                                                          const AxisArgs& ax, const SolveArgs& sa, int tx, int ty,
-                                                          int blk, float2* sm, int hxd) {
-  switch (code) {
-#define PME_F4_CASE(c, a, b)                                                                          \
-  case c:                                                                                             \
-    if constexpr (f4_class_of(a, b) == CLS)                                                              \
-      zsolve_four_step<a, b>(cg, hx, TX, pt_stride, outer_stride, ax, sa, tx, ty, blk, sm, hxd);      \
-    break;
-    PME_F4_PAIRS(PME_F4_CASE)
-#undef PME_F4_CASE
-    default: break;
-  }
-}
-
 // One tile of a y pass (S = -1 forward, +1 inverse) as a register four-step
 // with n = N1 N2 in ONE LDS buffer: the first half loads its columns
 // j2 + N2 j1 from HBM into registers, the second half reads its N2 points
@@ -1016,18 +587,6 @@ __device__ __forceinline__ void cols_four_step_dispatch(int code, float2* __rest
     default: break;
   }
 }
-
-// The fused z pass of one grid as a register four-step with n = N1 N2 (one
-// kernel per pair, so each gets the registers of its own pair only): column
-// tiles of TX lines of the flattened (ky, kx) of a z plane.
-template <int N1, int N2>
-__global__ __launch_bounds__(kBlock) void k_zsolve(float2* __restrict__ cg, int nlines, int TX, long long pt_stride,
-                                                   AxisArgs ax, SolveArgs sa, EvReduce red, int hxd) {
-  extern __shared__ __align__(16) float2 sm[];
-  if ((red.nsolve > 0 || red.nself > 0) && blockIdx.x == 0) ev_reduce_block<kBlock>(red);
-  zsolve_four_step<N1, N2>(cg, nlines, TX, pt_stride, 0, ax, sa, blockIdx.x, 0, blockIdx.x, sm, hxd);
-}
-
 
 // ------------------------------------------------------------ y / z passes --
 
@@ -1104,8 +663,8 @@ __global__ __launch_bounds__(kBlock) void k_fft_cols(float2* __restrict__ cg, in
 }
 
 // Stand-alone scalar sum over the whole half spectrum (used when the spectrum
-// has been materialised, e.g. scalar_sum called twice, and for triclinic
-// boxes).
+// has been materialised, e.g. scalar_sum called twice, and for a triclinic box
+// whose z length has no four-step pair or runs in split precision).
 __global__ __launch_bounds__(kBlock) void k_scalar_sum(float2* __restrict__ cg, int hx, int total, SolveArgs sa) {
   __shared__ double sh_red[7 * (kBlock / 64)];
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -1154,19 +713,11 @@ hipError_t launch_fft_cols(int mode, float2* cg, int n, int hx, int TX, long lon
   const size_t lds = fft_cols_lds_bytes(n, TX, four_step ? 1 : 2);
   const dim3 grid((hx + TX - 1) / TX, nouter);
   // the fused z pass indexes its tile with shifts
+  if (mode == COL_FWD_SOLVE_INV && sa.tric && !four_step) return hipErrorInvalidValue;  // no such kernel
   if (mode == COL_FWD_SOLVE_INV && (TX <= 0 || (TX & (TX - 1)) != 0)) return hipErrorInvalidValue;
   if (four_step) {
     if (nouter != 1 || outer_stride != 0) return hipErrorInvalidValue;  // one flattened plane of lines
-    switch (ax.f4) {
-#define PME_ZS_CASE(c, a, b)                                                                                       \
-  case c:                                                                                                          \
-    hipLaunchKernelGGL((k_zsolve<a, b>), grid, dim3(kBlock), lds, s, cg, hx, TX, pt_stride, ax, sa, red, hxd); \
-    break;
-      PME_F4_PAIRS(PME_ZS_CASE)
-#undef PME_ZS_CASE
-      default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return launch_zsolve(cg, hx, TX, pt_stride, ax, sa, red, hxd, lds, s);
   }
 #define PME_COLS(M)                                                                                         \
   if (split)                                                                                              \
@@ -1233,22 +784,6 @@ __global__ __launch_bounds__(kBlock) void k_batch_cols(const SysDesc* __restrict
   }
 }
 
-// The fused z pass of systems whose z length has a four-step pair of class
-// CLS (their items only): tiles of the flattened (ky, kx) of a z plane.
-template <int CLS>
-__global__ __launch_bounds__(kBlock, 4) void k_batch_zsolve(const SysDesc* __restrict__ sys,
-                                                         const WorkItem* __restrict__ items, int nitems) {
-  extern __shared__ __align__(16) float2 sm[];
-  for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
-    const WorkItem w = uniform_item(items[it]);
-    const SysDesc& d = sys[w.sys];
-    const int hx = d.bin.nx / 2 + 1;
-    zsolve_four_step_dispatch<CLS>(d.ax[2].f4, d.cgrid, hx * d.bin.ny, d.TXz, spec_pitch(hx, d.bin.ny), 0, d.ax[2],
-                                   d.sa, w.idx, 0, w.idx, sm, hx);
-    __syncthreads();
-  }
-}
-
 // items are (system, first plane z); each covers planes z .. z+g-1 with g =
 // plane_group(.., maxnp, NT < kPlaneBlock) of its system (fewer at the top of
 // the grid).  SPLIT: every system of the launch may use the matrix-core stage
@@ -1306,18 +841,6 @@ hipError_t launch_batch_fft_x(int inverse, const SysDesc* sys, const WorkItem* i
     hipLaunchKernelGGL(k_batch_fft_x<1>, dim3(grid), dim3(kBlock), lds, s, sys, items, nitems);
   else
     hipLaunchKernelGGL(k_batch_fft_x<0>, dim3(grid), dim3(kBlock), lds, s, sys, items, nitems);
-  return hipGetLastError();
-}
-
-hipError_t launch_batch_zsolve(int cls, const SysDesc* sys, const WorkItem* items, int nitems, int grid, size_t lds,
-                               hipStream_t s) {
-  if (nitems <= 0) return hipSuccess;
-  if (cls == 0)
-    hipLaunchKernelGGL(k_batch_zsolve<0>, dim3(grid), dim3(kBlock), lds, s, sys, items, nitems);
-  else if (cls == 1)
-    hipLaunchKernelGGL(k_batch_zsolve<1>, dim3(grid), dim3(kBlock), lds, s, sys, items, nitems);
-  else
-    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

@@ -276,6 +276,7 @@ struct pme_recip_s {
   hipEvent_t flush_ev = nullptr;
 
   int state = ST_EMPTY;
+  bool zinv_tric = false;     // ST_SOLVED_ZINV of a triclinic box
   const void* bin_key_ptr = nullptr;
   int bin_key_n = -1;
   float bin_key_r[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // (float) recip of the last binning
@@ -714,6 +715,18 @@ static pme_status z_pass(pme_recip_t h, int mode, const SolveArgs& sa) {
   return PME_OK;
 }
 
+// The z forward pass that completes the spectrum from the ST_XY or
+// ST_SOLVED_ZINV state.  After a triclinic solve the inverse and this forward
+// transform are undone to the spectrum as the stand-alone scalar sum leaves it
+// (an orthorhombic one carries the factor nz of the two transforms).
+static pme_status z_spectrum(pme_recip_t h) {
+  SolveArgs dummy{};
+  PME_TRY(z_pass(h, COL_FWD, dummy));
+  if (h->state == ST_SOLVED_ZINV && h->zinv_tric)
+    HIP_TRY(launch_scale_spectrum(h->cgrid, h->nx / 2 + 1, h->ny, h->nz, (float)(1.0 / h->nz), h->stream));
+  return PME_OK;
+}
+
 extern "C" pme_status pme_recip_scalar_sum(pme_recip_t h, const double recip[9], double kappa, int calc_energy,
                                            int calc_virial) {
   if (!h || !recip) return fail(PME_ERR_INVALID_ARG, "pme_recip_scalar_sum: null argument");
@@ -727,14 +740,15 @@ extern "C" pme_status pme_recip_scalar_sum(pme_recip_t h, const double recip[9],
   SolveArgs sa = solve_args(h, recip, kappa, ev);
   const int hx = h->nx / 2 + 1;
   mark(h, 4);
-  if (h->state == ST_XY && !sa.tric) {
+  if (h->state == ST_XY && (!sa.tric || axis_args(h, 2).f4 >= 0)) {
     PME_TRY(z_pass(h, COL_FWD_SOLVE_INV, sa));
     if (ev) h->pend_solve = cols_blocks(hx * h->ny, h->TXz, 1);
     h->state = ST_SOLVED_ZINV;
+    h->zinv_tric = sa.tric != 0;
   } else {
-    // the spectrum in full first (a triclinic box: the fused z pass holds
-    // the orthorhombic influence function only)
-    if (h->state == ST_SOLVED_ZINV || h->state == ST_XY) PME_TRY(z_pass(h, COL_FWD, sa));
+    // the spectrum in full first (a triclinic box: the Stockham and split z
+    // passes hold the orthorhombic influence function only)
+    if (h->state == ST_SOLVED_ZINV || h->state == ST_XY) PME_TRY(z_spectrum(h));
     HIP_TRY(launch_scalar_sum(h->cgrid, hx, sa, h->stream));
     if (ev) h->pend_solve = scalar_sum_blocks(hx * h->ny * h->nz);
     h->state = ST_SPECTRUM;
@@ -1074,8 +1088,7 @@ extern "C" pme_status pme_recip_copy_grid(pme_recip_t h, int which, void* d_dst,
     HIP_TRY(hipMemcpyAsync(d_dst, h->grid, G * sizeof(float), hipMemcpyDeviceToDevice, h->stream));
   } else if (which == PME_GRID_SPECTRUM) {
     if (h->state == ST_XY || h->state == ST_SOLVED_ZINV) {
-      SolveArgs dummy{};
-      PME_TRY(z_pass(h, COL_FWD, dummy));
+      PME_TRY(z_spectrum(h));
       h->state = ST_SPECTRUM;
     }
     if (h->state != ST_SPECTRUM) return fail(PME_ERR_STATE, "pme_recip_copy_grid: no spectrum");

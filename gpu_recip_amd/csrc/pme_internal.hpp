@@ -90,7 +90,7 @@ struct SolveArgs {
   int calc_ev;             // accumulate energy and virial
   double* partial;         // [nblocks * 7] per-workgroup partial sums
   float rt[9];             // (float) recip, row-major, for a triclinic box
-  int tric;                // 1: m-hat from the full recip (stand-alone scalar sum only)
+  int tric;                // 1: m-hat from the full recip (four-step z pass and stand-alone scalar sum)
 };
 
 enum ColMode { COL_FWD = 0, COL_INV = 1, COL_FWD_SOLVE_INV = 2, COL_FWD_INV = 3 };
@@ -241,6 +241,11 @@ hipError_t launch_fft_cols(int mode, float2* cg, int n, int hx, int TX, long lon
                            int nouter, long long outer_stride, const AxisArgs& ax,
                            const SolveArgs& sa, const EvReduce& red, int hxd, hipStream_t s);
 int cols_blocks(int hx, int TX, int nouter);
+// the fused z pass of a length with a four-step pair (pme_zsolve.hip), sa.tric included
+hipError_t launch_zsolve(float2* cg, int nlines, int TX, long long pt_stride, const AxisArgs& ax, const SolveArgs& sa,
+                         const EvReduce& red, int hxd, size_t lds, hipStream_t s);
+// every point of the half spectrum times f
+hipError_t launch_scale_spectrum(float2* cg, int hx, int ny, int nz, float f, hipStream_t s);
 hipError_t launch_scalar_sum(float2* cg, int hx, const SolveArgs& sa, hipStream_t s);
 int scalar_sum_blocks(int total);
 
@@ -331,7 +336,7 @@ bool four_step_pair(int code, int* n1, int* n2);
 // four_step_code of a radix plan's four-step pair when the table holds that
 // pair, else -1 (the y passes then run the generic stages)
 int four_step_code_for_plan(const RadixPlan& rp);
-// register class of a four-step pair (0: N2 <= 10 and 5 x 15, 1: the others), -1: none
+// register class of a four-step pair (0: N2 <= 10 and 5 x 15, 1: N2 <= 16, 2: longer), -1: none
 int four_step_class(int code);
 
 // LDS bytes of a plane kernel over np planes per workgroup (0 when they do

@@ -296,7 +296,7 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
   for (int sp : {0, 1}) add_stage(BS_FFTY, 0, sp, 0);
   for (int sp : {0, 1, 2})
     for (int h : {1, 0}) add_stage(BS_PLANE, group, sp, h);
-  for (int c : {1, 2}) add_stage(BS_FFTZ, c, 0, 0);
+  for (int c : {1, 2, 3}) add_stage(BS_FFTZ, c, 0, 0);
   for (int sp : {0, 1}) add_stage(BS_FFTZ, 0, sp, 0);
   for (int o : {4, 6, 8}) add_stage(BS_GATHER, o, 0, 0);
 }
