@@ -139,6 +139,14 @@ __device__ __forceinline__ int brick_of(int i, int n, int nb) { return ((i + 1) 
 // ---- complex helpers -----------------------------------------------------
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+// A complex value stored at agent scope: written through the XCD's L2 at once
+// instead of left dirty there and written back when the kernel ends, which the
+// next kernel waits for.  For stores in whole contiguous runs.
+__device__ __forceinline__ void store_through(float2* g, float2 v) {
+  const unsigned long long u =
+      (unsigned long long)__float_as_uint(v.x) | ((unsigned long long)__float_as_uint(v.y) << 32);
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(g), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
