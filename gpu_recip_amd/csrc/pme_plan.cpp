@@ -120,10 +120,11 @@ std::vector<float2> twiddles(int n) {
   return t;
 }
 
-bool plan_bricks(const int n[3], int order, int target, BrickPlan* bp, size_t budget) {
+bool plan_bricks(const int n[3], int order, int target, BrickPlan* bp, size_t budget, const int* extra) {
   for (int a = 0; a < 3; a++) {
     int nb = (n[a] + target / 2) / target;
     if (nb < 1) nb = 1;
+    if (extra) nb += extra[a];
     while (nb > 1 && n[a] / nb < order - 1) nb--;
     bp->nb[a] = nb;
     bp->wmax[a] = (n[a] + nb - 1) / nb;
@@ -150,6 +151,8 @@ bool plan_bricks(const int n[3], int order, int target, BrickPlan* bp, size_t bu
 // scale alike.  It ranks the measured plans right: at 96k atoms brick 16
 // (99.9 us per solve) ahead of 18/20/24 (105.8/116.9/124.1), at 250,002 atoms,
 // 144^3, order 4 brick 24 (145.2) ahead of 18/20/16 (149.1/157.3/161.2).
+// A brick of a small grid costs less than the model's (8,001 atoms, 48^3: 6.6 us a
+// launch at brick 8, 8.5 at 16), which does not change the choice.
 static double brick_cost(const int n[3], int order, int ncu, const BrickPlan& bp) {
   const double g = (double)n[0] * n[1] * n[2];
   const double pts = g / bp.nbins;
@@ -160,19 +163,27 @@ static double brick_cost(const int n[3], int order, int ncu, const BrickPlan& bp
   return rounds * (7.7 + pts * (8.3e-4 + 1.59e-3 * halo * p3));
 }
 
+// The plans weighed are those of the targets, and of each target with one more
+// brick along y, z or both (x keeps its rows): a cubic count leaves up to a
+// third of the CUs idle (144^3, order 4, 216 -> 252 bricks: spread 18.7 -> 17.9 us,
+// gather 17.3 -> 16.2).  Targets below 16 are for grids with fewer bricks of 16
+// than CUs (23,559 atoms, 64^3, order 6, 64 -> 252 bricks: spread 17.6 -> 13.6, gather
+// 12.2 -> 9.6; 2,001 atoms, 32^3, order 4, 8 -> 64 bricks: 7.7 -> 6.3, 6.9 -> 5.9).
 bool plan_bricks_auto(const int n[3], int order, int ncu, BrickPlan* bp) {
   bool any = false;
   double best = 0.0;
-  for (int target : {16, 18, 20, 24, 28, 32}) {
-    BrickPlan t;
-    if (!plan_bricks(n, order, target, &t)) continue;
-    const double c = brick_cost(n, order, std::max(ncu, 1), t);
-    if (!any || c < best) {
-      best = c;
-      *bp = t;
-      any = true;
+  for (int target : {8, 10, 12, 14, 16, 18, 20, 24, 28, 32})
+    for (int more = 0; more < 4; more++) {
+      BrickPlan t;
+      const int extra[3] = {0, more >> 1, more & 1};
+      if (!plan_bricks(n, order, target, &t, kBrickLdsBudget, extra)) continue;
+      const double c = brick_cost(n, order, std::max(ncu, 1), t);
+      if (!any || c < best) {
+        best = c;
+        *bp = t;
+        any = true;
+      }
     }
-  }
   return any;
 }
 
