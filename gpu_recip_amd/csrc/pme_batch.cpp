@@ -376,7 +376,7 @@ static pme_status enqueue(pme_batch_t b) {
   }
   const int n = (int)b->slots.size();
   if (n > 0)
-    BHIP(hipMemcpyAsync(b->h_ev, b->d_ev, sizeof(double) * kEvOut * (size_t)n, hipMemcpyDeviceToHost, b->stream));
+    BHIP(launch_copy_words(b->h_ev, b->d_ev, sizeof(double) * kEvOut * (size_t)n, nullptr, nullptr, 0, b->stream));
   b->ev_copied = n;
   return PME_OK;
 }

@@ -254,6 +254,10 @@ hipError_t launch_ev_reduce(const EvReduce& red, hipStream_t s);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s);
 // pending reduction red, then device buffer to pinned host memory (whole 8-byte words)
 hipError_t launch_copy_out(void* host, const void* dev, size_t bytes, const EvReduce& red, hipStream_t s);
+// dst0 <- src0 and dst1 <- src1 (bytes multiples of 8, either may be 0), device or
+// pinned host memory
+hipError_t launch_copy_words(void* dst0, const void* src0, size_t bytes0, void* dst1, const void* src1, size_t bytes1,
+                             hipStream_t s);
 hipError_t launch_fill_bspline(int order, const float4* xyzq, int n, float r1, float r2, float r3,
                                int nx, int ny, int nz, int* gix, int* giy, int* giz, float* q,
                                float* thx, float* thy, float* thz, float* dthx, float* dthy,

@@ -293,13 +293,12 @@ static pme_status launch_lane(pme_server_t s, Lane& L, std::vector<Request>& sel
   for (const Request& r : sel)
     if (r.ready && hipStreamWaitEvent(L.stream, r.ready, 0) != hipSuccess)
       return set_error(PME_ERR_DEVICE, "hipStreamWaitEvent on a ready event");
-  if (hipMemcpyAsync(L.d_sys, L.h_stage, sizeof(SysDesc) * m, hipMemcpyHostToDevice, L.stream) != hipSuccess ||
-      hipMemcpyAsync(L.d_items, L.h_stage + sizeof(SysDesc) * L.cap_sys, sizeof(WorkItem) * items.size(),
-                     hipMemcpyHostToDevice, L.stream) != hipSuccess)
+  if (launch_copy_words(L.d_sys, L.h_stage, sizeof(SysDesc) * m, L.d_items, L.h_stage + sizeof(SysDesc) * L.cap_sys,
+                        sizeof(WorkItem) * items.size(), L.stream) != hipSuccess)
     return set_error(PME_ERR_DEVICE, "serving lane upload");
   st = enqueue_stages(launches, L.d_sys, L.d_items, tune, s->ncu, L.stream, nullptr);
   if (st != PME_OK) return st;
-  if (hipMemcpyAsync(L.h_ev, L.d_ev, sizeof(double) * kEvOut * m, hipMemcpyDeviceToHost, L.stream) != hipSuccess ||
+  if (launch_copy_words(L.h_ev, L.d_ev, sizeof(double) * kEvOut * m, nullptr, nullptr, 0, L.stream) != hipSuccess ||
       hipEventRecord(L.done, L.stream) != hipSuccess)
     return set_error(PME_ERR_DEVICE, "serving lane readback");
   for (const Request& r : sel) s->resident[r.key].busy = true;
