@@ -692,7 +692,7 @@ extern "C" pme_status pme_recip_r2c_fft(pme_recip_t h) {
   mark(h, 2);
   const AxisArgs ax = axis_args(h, 0), ay = axis_args(h, 1);
   const PlaneKind plane = plane_kind(h->nx, h->ny, ax.rp, ay.rp, ay.prec);
-  if (plane == PLANE_FOUR_STEP) {
+  if (plane_is_four_step(plane)) {
     HIP_TRY(launch_plane4_fwd(h->grid, h->cgrid, h->nx, h->ny, h->nz, ax, ay, h->stream));
     mark(h, 3);
   } else if (plane == PLANE_STAGES) {
@@ -773,7 +773,7 @@ extern "C" pme_status pme_recip_c2r_fft(pme_recip_t h) {
   const AxisArgs ax = axis_args(h, 0), ay = axis_args(h, 1);
   const PlaneKind plane = plane_kind(h->nx, h->ny, ax.rp, ay.rp, ay.prec);
   if (plane != PLANE_NONE) {
-    if (plane == PLANE_FOUR_STEP)
+    if (plane_is_four_step(plane))
       HIP_TRY(launch_plane4_inv(h->cgrid, h->grid, h->nx, h->ny, h->nz, ax, ay, pending_reduce(h), h->stream));
     else
       HIP_TRY(launch_fft_plane_inv(h->cgrid, h->grid, h->nx, h->ny, h->nz, ax, ay, pending_reduce(h), h->stream));

@@ -117,8 +117,10 @@ struct SysDesc {
   double kcs;              // kappa*ccelec/sqrt(pi)
 };
 // x and y passes: separate kernels, one xy plane kernel in Stockham or
-// matrix-core stages (two LDS buffers), or as register four-steps (one buffer)
-enum PlaneKind { PLANE_NONE = 0, PLANE_STAGES = 1, PLANE_FOUR_STEP = 2 };
+// matrix-core stages (two LDS buffers), or as register four-steps (one buffer),
+// with FP32 or split-precision 16-point DFTs in y
+enum PlaneKind { PLANE_NONE = 0, PLANE_STAGES = 1, PLANE_FOUR_STEP = 2, PLANE_FOUR_STEP_SPLIT = 3 };
+constexpr bool plane_is_four_step(int kind) { return kind == PLANE_FOUR_STEP || kind == PLANE_FOUR_STEP_SPLIT; }
 constexpr int kEvOut = 11;  // doubles per system in the batched energy/virial output
 
 // One workgroup-sized task of a batched stage: system index and the tile of
@@ -362,7 +364,7 @@ hipError_t launch_batch_plane(int inverse, int reduce, int maxnp, int split, int
                               const WorkItem* items, int nitems, int grid, size_t lds, hipStream_t s);
 
 // Plane kernels as register four-steps (pme_plane.hip): both lengths have a
-// four-step pair (plane4_ok) and FP32 axes.
+// four-step pair (FP32 y axis: plane4_ok).
 bool plane4_ok(const RadixPlan& rx, const RadixPlan& ry);
 size_t fft_plane4_lds_bytes(int nx, int ny, int np);  // 0: does not fit one workgroup
 int plane4_group_host(int nx, int ny, int maxnp, bool half);
@@ -371,8 +373,8 @@ hipError_t launch_plane4_fwd(const float* grid, float2* cg, int nx, int ny, int 
                              const AxisArgs& ay, hipStream_t s);
 hipError_t launch_plane4_inv(const float2* cg, float* grid, int nx, int ny, int nz, const AxisArgs& ax,
                              const AxisArgs& ay, const EvReduce& red, hipStream_t s);
-hipError_t launch_batch_plane4(int inverse, int reduce, int maxnp, int half, const SysDesc* sys, const WorkItem* items,
-                               int nitems, int grid, size_t lds, hipStream_t s);
+hipError_t launch_batch_plane4(int inverse, int reduce, int maxnp, int split, int half, const SysDesc* sys,
+                               const WorkItem* items, int nitems, int grid, size_t lds, hipStream_t s);
 // how the x and y passes of a grid run (y_prec: PREC_* of the y axis)
 PlaneKind plane_kind(int nx, int ny, const RadixPlan& rx, const RadixPlan& ry, int y_prec);
 

@@ -22,6 +22,12 @@
 // pair split mixes rows, so the spectrum columns have a buffer of their own).
 // A plane of 144 x 144 takes 84 KB of the 160 KB LDS.
 //
+// A split-precision y axis of 16 b points (b a codelet length up to 12) takes
+// DFT_Ay = 16 and DFT_By = b in both directions and runs the 16-point DFTs on the
+// matrix cores (SPLIT).  They come first forward too: after the other factor their
+// columns mix large and small frequencies, and the hi-lo error, which goes with the
+// column's largest, was 15 % more in the forces.
+//
 // Bound by the VALU and the LDS round trips, not by HBM (the two launches of
 // the 108 x 100 x 96 grid move 16 MB).  LDS points are line-minor (point p of
 // line l at p * LS + l, LS odd): lanes run along lines in the passes that
@@ -81,13 +87,22 @@ size_t plane4_lds_need(int nx, int ny, int np) {
 
 bool plane4_ok(const RadixPlan& rx, const RadixPlan& ry) { return rx.f4a > 0 && ry.f4a > 0 && ry.f4a <= PME_PL_PAIR_MAX; }
 
+// split-precision y axis: 16 b with the 16-point DFTs on the matrix cores, b
+// the smaller factor's codelet
+static bool plane4_split_ok(const RadixPlan& rx, const RadixPlan& ry) {
+  return rx.f4a > 0 && ry.f4a == 16 && ry.f4b > 0 && ry.f4b <= PME_PL_PAIR_MAX;
+}
+
 size_t fft_plane4_lds_bytes(int nx, int ny, int np) {
   const size_t b = plane4_lds_need(nx, ny, np);
   return b <= kPlaneLdsBudget ? b : 0;
 }
 
 PlaneKind plane_kind(int nx, int ny, const RadixPlan& rx, const RadixPlan& ry, int y_prec) {
-  if (y_prec == PREC_FP32 && plane4_ok(rx, ry) && fft_plane4_lds_bytes(nx, ny, 1)) return PLANE_FOUR_STEP;
+  if (fft_plane4_lds_bytes(nx, ny, 1)) {
+    if (y_prec == PREC_FP32 && plane4_ok(rx, ry)) return PLANE_FOUR_STEP;
+    if (y_prec != PREC_FP32 && plane4_split_ok(rx, ry)) return PLANE_FOUR_STEP_SPLIT;
+  }
   return fft_plane_lds_bytes(nx, ny, rx.n, 1) ? PLANE_STAGES : PLANE_NONE;
 }
 
@@ -282,6 +297,90 @@ __device__ __forceinline__ void pl_fwd_pair(const float2* b, float2* d, const fl
   }
 }
 
+// pass 3 with the DFT_16 as hi-lo products on the matrix cores, even nx: 32
+// columns per wave are 16 units (pair, plane, j2), lanes j and j + 16 columns k and
+// h-k of one unit, each forming its own column of the split as it loads.  In place:
+// a wave has loaded all its columns before it stores the first.
+template <int PREC, int NT>
+__device__ __forceinline__ void pl_fwd_split_mfma(float2* b, const float2* twx, const float2* twy, int B, int Ax,
+                                                  int Bx, const PlaneGeo& g) {
+  const SmallDiv dB = small_div(B), dnp = small_div(g.np), dax = small_div(Ax);
+  const int n = mul24(mul24((g.h >> 1) + 1, g.np), B);
+  struct Ctx {
+    const float2 *z, *zc;  // Z[k], Z[h-k] of row j2 (of the lane's own column k)
+    float2* out;           // null: nothing to store
+    float2 w;
+    int j2;
+  };
+  mfma_dft16_cols<-1, PREC>(
+      32 * ((n + 15) >> 4),
+      [&](int u) {
+        const int v = (u >> 5) * 16 + (u & 15);
+        const bool live = v < n, second = (u & 16) != 0;
+        const int t = sdiv(live ? v : 0, dB);
+        const int j2 = (live ? v : 0) - mul24(t, B);
+        const int k = sdiv(t, dnp);
+        const int r = mul24(t - mul24(k, g.np), g.ny) + j2;
+        const int c = g.h - k;
+        const int qk = sdiv(k, dax), qc = sdiv(c, dax);
+        float2* pk = b + (mul24(mul24(k - mul24(qk, Ax), Bx) + qk, g.LX) + r);
+        float2* pc = b + (mul24(k == 0 ? g.h : mul24(c - mul24(qc, Ax), Bx) + qc, g.LX) + r);
+        float2* pz = k == 0 ? pk : pc;
+        Ctx x;
+        x.z = pk;
+        x.zc = pz;
+        x.out = live && !(second && c == k) ? (second ? pc : pk) : nullptr;
+        x.w = twx[k];
+        x.j2 = second ? -1 - j2 : j2;  // sign: which column of the pair
+        return x;
+      },
+      [&](const Ctx& x, int m) {
+        const float2 zk = x.z[mul24(m, B)], zc = cconj(x.zc[mul24(m, B)]);
+        const float2 E = cscale(cadd(zk, zc), 0.5f);
+        const float2 D = csub(zk, zc);
+        const float2 T = cmul(x.w, make_float2(0.5f * D.y, -0.5f * D.x));
+        return x.j2 < 0 ? cconj(csub(E, T)) : cadd(E, T);
+      },
+      [&](const Ctx& x, int q, float2 y) {
+        if (x.out) x.out[mul24(q, B)] = q == 0 ? y : cmul(y, twy[mul24(q, x.j2 < 0 ? -1 - x.j2 : x.j2)]);
+      },
+      threadIdx.x, NT);
+}
+
+// the same for odd nx: units (column k, plane, j2), into the column buffer
+template <int PREC, int NT>
+__device__ __forceinline__ void pl_fwd_pair_mfma(const float2* b, float2* d, const float2* twy, int B, int Ax, int Bx,
+                                                 const PlaneGeo& g) {
+  const SmallDiv dB = small_div(B), dnp = small_div(g.np), dax = small_div(Ax);
+  const int hyl = (g.ny + 1) >> 1;
+  struct Ctx {
+    const float2 *z, *zc;
+    float2* out;
+    int j2;
+  };
+  mfma_dft16_cols<-1, PREC>(
+      mul24(mul24(g.hx, g.np), B),
+      [&](int u) {
+        const int t = sdiv(u, dB);
+        const int j2 = u - mul24(t, B);
+        const int k = sdiv(t, dnp);
+        const int pl = t - mul24(k, g.np);
+        const int c = k == 0 ? 0 : g.nx - k;
+        const int qk = sdiv(k, dax), qc = sdiv(c, dax);
+        return Ctx{b + (mul24(mul24(k - mul24(qk, Ax), Bx) + qk, g.LX) + mul24(pl, hyl)),
+                   b + (mul24(mul24(c - mul24(qc, Ax), Bx) + qc, g.LX) + mul24(pl, hyl)),
+                   d + (mul24(k, g.LY) + mul24(pl, g.ny) + j2), j2};
+      },
+      [&](const Ctx& x, int m) {
+        const int y = x.j2 + mul24(m, B);
+        const float2 zk = x.z[y >> 1], zc = cconj(x.zc[y >> 1]);
+        const float2 D = csub(zk, zc);
+        return (y & 1) ? make_float2(0.5f * D.y, -0.5f * D.x) : cscale(cadd(zk, zc), 0.5f);
+      },
+      [&](const Ctx& x, int q, float2 y) { x.out[mul24(q, B)] = q == 0 ? y : cmul(y, twy[mul24(q, x.j2)]); },
+      threadIdx.x, NT);
+}
+
 // pass 4: unit (k1, plane, column k), columns fastest: DFT_B over the row
 // positions k1 B + j2, Y[k1 + A k2] stored to the half-spectrum planes
 // (column k at slot (k mod Ax) Bx + k / Ax; Ax = 1: at k).  Written through the
@@ -311,7 +410,7 @@ __device__ __forceinline__ void pl_fwd_store(const float2* b, float2* __restrict
   }
 }
 
-template <int NT>
+template <int NT, bool SPLIT>
 __device__ __forceinline__ void plane4_fwd_body(const float* __restrict__ grid, float2* __restrict__ cg, int nx,
                                                 int ny, const AxisArgs& axx, const AxisArgs& axy, int z, int np,
                                                 float2* sm) {
@@ -321,7 +420,8 @@ __device__ __forceinline__ void plane4_fwd_body(const float* __restrict__ grid, 
   float2* b = twy + ny;
   for (int i = threadIdx.x; i < nx; i += NT) twx[i] = axx.tw[i];
   for (int i = threadIdx.x; i < ny; i += NT) twy[i] = axy.tw[i];
-  const int Ax = axx.rp.f4a, Bx = axx.rp.f4b, Ay = axy.rp.f4a, By = axy.rp.f4b;
+  const int Ax = axx.rp.f4a, Bx = axx.rp.f4b;
+  const int Ay = axy.rp.f4a, By = axy.rp.f4b;  // SPLIT: Ay = 16
   const float* src = grid + (size_t)z * nx * ny;
 #define PME_CALL(L) \
   case L: pl_fwd_load<L, NT>(src, b, twx, axx.rp.tstride, Bx, g); break;
@@ -333,14 +433,25 @@ __device__ __forceinline__ void plane4_fwd_body(const float* __restrict__ grid, 
   PME_PL_SWITCH(Bx, PME_CALL)
 #undef PME_CALL
   __syncthreads();
-  float2* d = b;
-  if (!g.odd) {
+  float2* d = g.odd ? b + g.bx : b;
+  if constexpr (SPLIT) {
+    if (g.odd) {
+      if (axy.prec == PREC_BF16X3)
+        pl_fwd_pair_mfma<PREC_BF16X3, NT>(b, d, twy, By, Ax, Bx, g);
+      else
+        pl_fwd_pair_mfma<PREC_FP16X3, NT>(b, d, twy, By, Ax, Bx, g);
+    } else {
+      if (axy.prec == PREC_BF16X3)
+        pl_fwd_split_mfma<PREC_BF16X3, NT>(b, twx, twy, By, Ax, Bx, g);
+      else
+        pl_fwd_split_mfma<PREC_FP16X3, NT>(b, twx, twy, By, Ax, Bx, g);
+    }
+  } else if (!g.odd) {
 #define PME_CALL(L) \
   case L: pl_fwd_split<L, NT>(b, twx, twy, By, Ax, Bx, g); break;
     PME_PL_PAIR_SWITCH(Ay, PME_CALL)
 #undef PME_CALL
   } else {
-    d = b + g.bx;
 #define PME_CALL(L) \
   case L: pl_fwd_pair<L, NT>(b, d, twy, By, Ax, Bx, g); break;
     PME_PL_PAIR_SWITCH(Ay, PME_CALL)
@@ -387,6 +498,35 @@ __device__ __forceinline__ void pl_inv_load(const float2* __restrict__ src, floa
       for (int q = 1; q < A; q++) p[mul24(q, B)] = cmulc(x[q], tw[mul24(q, j2)]);
     }
   }
+}
+
+// pass 1 with the DFT_16 as hi-lo products on the matrix cores: units (j2,
+// plane, column), 32 of them per wave
+template <int PREC, int NT>
+__device__ __forceinline__ void pl_inv_load_split(const float2* __restrict__ src, float2* b, const float2* tw, int B,
+                                                  const PlaneGeo& g, long long pz) {
+  const int ncol = mul24(g.np, g.hx);
+  const SmallDiv dnc = small_div(ncol), dhx = small_div(g.hx);
+  const int st = mul24(B, g.hx);
+  struct Ctx {
+    const float2* s;
+    float2* p;
+    int j2;
+  };
+  __syncthreads();  // twiddles in LDS
+  mfma_dft16_cols<1, PREC>(
+      B * ncol,
+      [&](int u) {
+        const int j2 = sdiv(u, dnc);
+        const int c = u - mul24(j2, ncol);
+        const int pl = sdiv(c, dhx);
+        const int k = c - mul24(pl, g.hx);
+        return Ctx{src + ((size_t)pl * (size_t)pz + (mul24(j2, g.hx) + k)),
+                   b + (mul24(k, g.LY) + mul24(pl, g.ny) + j2), j2};
+      },
+      [&](const Ctx& x, int m) { return x.s[mul24(m, st)]; },
+      [&](const Ctx& x, int q, float2 y) { x.p[mul24(q, B)] = q == 0 ? y : cmulc(y, tw[mul24(q, x.j2)]); },
+      threadIdx.x, NT);
 }
 
 // pass 2, even nx: unit (pair k <= h/2, plane, k1), k1 fastest: DFT_B of
@@ -526,7 +666,7 @@ __device__ __forceinline__ void pl_inv_store(const float2* b, float* __restrict_
   }
 }
 
-template <int NT>
+template <int NT, bool SPLIT>
 __device__ __forceinline__ void plane4_inv_body(const float2* __restrict__ cg, float* __restrict__ grid, int nx,
                                                 int ny, const AxisArgs& axx, const AxisArgs& axy, int z, int np,
                                                 float2* sm) {
@@ -536,14 +676,22 @@ __device__ __forceinline__ void plane4_inv_body(const float2* __restrict__ cg, f
   float2* b = twy + ny;
   for (int i = threadIdx.x; i < nx; i += NT) twx[i] = axx.tw[i];
   for (int i = threadIdx.x; i < ny; i += NT) twy[i] = axy.tw[i];
-  const int Ax = axx.rp.f4b, Bx = axx.rp.f4a, Ay = axy.rp.f4b, By = axy.rp.f4a;
+  const int Ax = axx.rp.f4b, Bx = axx.rp.f4a;
+  const int Ay = SPLIT ? 16 : axy.rp.f4b, By = SPLIT ? axy.rp.f4b : axy.rp.f4a;
   const long long pz = spec_pitch(g.hx, ny);
   const float2* src = cg + (size_t)z * (size_t)pz;
   float2* d = g.odd ? b + g.bx : b;  // columns
+  if constexpr (SPLIT) {
+    if (axy.prec == PREC_BF16X3)
+      pl_inv_load_split<PREC_BF16X3, NT>(src, d, twy, By, g, pz);
+    else
+      pl_inv_load_split<PREC_FP16X3, NT>(src, d, twy, By, g, pz);
+  } else {
 #define PME_CALL(L) \
   case L: pl_inv_load<L, NT>(src, d, twy, By, g, pz); break;
-  PME_PL_SWITCH(Ay, PME_CALL)
+    PME_PL_SWITCH(Ay, PME_CALL)
 #undef PME_CALL
+  }
   __syncthreads();
   if (!g.odd) {
 #define PME_CALL(L) \
@@ -576,16 +724,16 @@ __device__ __forceinline__ void plane4_inv_body(const float2* __restrict__ cg, f
 
 // ---- kernels -----------------------------------------------------------------------
 
-template <int NT>
+template <int NT, bool SPLIT>
 __global__ __launch_bounds__(NT, 4) void k_plane4_fwd(const float* __restrict__ grid, float2* __restrict__ cg, int nx,
                                                       int ny, AxisArgs axx, AxisArgs axy) {
   extern __shared__ __align__(16) float2 sm[];
-  plane4_fwd_body<NT>(grid, cg, nx, ny, axx, axy, blockIdx.x, 1, sm);
+  plane4_fwd_body<NT, SPLIT>(grid, cg, nx, ny, axx, axy, blockIdx.x, 1, sm);
 }
 
 // With a pending energy/virial reduction the launch has one more workgroup
 // that performs it alone, so no plane's workgroup waits for it.
-template <int NT>
+template <int NT, bool SPLIT>
 __global__ __launch_bounds__(NT, 4) void k_plane4_inv(const float2* __restrict__ cg, float* __restrict__ grid, int nx,
                                                       int ny, int nz, AxisArgs axx, AxisArgs axy, EvReduce red) {
   extern __shared__ __align__(16) float2 sm[];
@@ -593,7 +741,7 @@ __global__ __launch_bounds__(NT, 4) void k_plane4_inv(const float2* __restrict__
     ev_reduce_block<NT>(red);
     return;
   }
-  plane4_inv_body<NT>(cg, grid, nx, ny, axx, axy, blockIdx.x, 1, sm);
+  plane4_inv_body<NT, SPLIT>(cg, grid, nx, ny, axx, axy, blockIdx.x, 1, sm);
 }
 
 // Threads of a single-system plane workgroup: one unit of work each in the
@@ -604,35 +752,57 @@ static int plane4_threads(int nx, int ny, const AxisArgs& ax, const AxisArgs& ay
   return u <= 256 ? 256 : (u <= 512 ? 512 : 1024);
 }
 
+template <bool SPLIT>
+static void plane4_fwd_as(const float* grid, float2* cg, int nx, int ny, int nz, const AxisArgs& ax,
+                          const AxisArgs& ay, size_t lds, hipStream_t s) {
+  switch (plane4_threads(nx, ny, ax, ay)) {
+    case 256: hipLaunchKernelGGL((k_plane4_fwd<256, SPLIT>), dim3(nz), dim3(256), lds, s, grid, cg, nx, ny, ax, ay); break;
+    case 512: hipLaunchKernelGGL((k_plane4_fwd<512, SPLIT>), dim3(nz), dim3(512), lds, s, grid, cg, nx, ny, ax, ay); break;
+    default: hipLaunchKernelGGL((k_plane4_fwd<1024, SPLIT>), dim3(nz), dim3(1024), lds, s, grid, cg, nx, ny, ax, ay); break;
+  }
+}
+
 hipError_t launch_plane4_fwd(const float* grid, float2* cg, int nx, int ny, int nz, const AxisArgs& ax,
                              const AxisArgs& ay, hipStream_t s) {
   const size_t lds = fft_plane4_lds_bytes(nx, ny, 1);
-  if (!lds || !plane4_ok(ax.rp, ay.rp)) return hipErrorInvalidValue;
-  switch (plane4_threads(nx, ny, ax, ay)) {
-    case 256: hipLaunchKernelGGL(k_plane4_fwd<256>, dim3(nz), dim3(256), lds, s, grid, cg, nx, ny, ax, ay); break;
-    case 512: hipLaunchKernelGGL(k_plane4_fwd<512>, dim3(nz), dim3(512), lds, s, grid, cg, nx, ny, ax, ay); break;
-    default: hipLaunchKernelGGL(k_plane4_fwd<1024>, dim3(nz), dim3(1024), lds, s, grid, cg, nx, ny, ax, ay); break;
-  }
+  const PlaneKind kind = plane_kind(nx, ny, ax.rp, ay.rp, ay.prec);
+  if (kind == PLANE_FOUR_STEP)
+    plane4_fwd_as<false>(grid, cg, nx, ny, nz, ax, ay, lds, s);
+  else if (kind == PLANE_FOUR_STEP_SPLIT)
+    plane4_fwd_as<true>(grid, cg, nx, ny, nz, ax, ay, lds, s);
+  else
+    return hipErrorInvalidValue;
   return hipGetLastError();
+}
+
+template <bool SPLIT>
+static void plane4_inv_as(const float2* cg, float* grid, int nx, int ny, int nz, const AxisArgs& ax,
+                          const AxisArgs& ay, const EvReduce& red, size_t lds, hipStream_t s) {
+  const dim3 gr(nz + ((red.nsolve > 0 || red.nself > 0) ? 1 : 0));
+  switch (plane4_threads(nx, ny, ax, ay)) {
+    case 256: hipLaunchKernelGGL((k_plane4_inv<256, SPLIT>), gr, dim3(256), lds, s, cg, grid, nx, ny, nz, ax, ay, red); break;
+    case 512: hipLaunchKernelGGL((k_plane4_inv<512, SPLIT>), gr, dim3(512), lds, s, cg, grid, nx, ny, nz, ax, ay, red); break;
+    default: hipLaunchKernelGGL((k_plane4_inv<1024, SPLIT>), gr, dim3(1024), lds, s, cg, grid, nx, ny, nz, ax, ay, red); break;
+  }
 }
 
 hipError_t launch_plane4_inv(const float2* cg, float* grid, int nx, int ny, int nz, const AxisArgs& ax,
                              const AxisArgs& ay, const EvReduce& red, hipStream_t s) {
   const size_t lds = fft_plane4_lds_bytes(nx, ny, 1);
-  if (!lds || !plane4_ok(ax.rp, ay.rp)) return hipErrorInvalidValue;
-  const dim3 gr(nz + ((red.nsolve > 0 || red.nself > 0) ? 1 : 0));
-  switch (plane4_threads(nx, ny, ax, ay)) {
-    case 256: hipLaunchKernelGGL(k_plane4_inv<256>, gr, dim3(256), lds, s, cg, grid, nx, ny, nz, ax, ay, red); break;
-    case 512: hipLaunchKernelGGL(k_plane4_inv<512>, gr, dim3(512), lds, s, cg, grid, nx, ny, nz, ax, ay, red); break;
-    default: hipLaunchKernelGGL(k_plane4_inv<1024>, gr, dim3(1024), lds, s, cg, grid, nx, ny, nz, ax, ay, red); break;
-  }
+  const PlaneKind kind = plane_kind(nx, ny, ax.rp, ay.rp, ay.prec);
+  if (kind == PLANE_FOUR_STEP)
+    plane4_inv_as<false>(cg, grid, nx, ny, nz, ax, ay, red, lds, s);
+  else if (kind == PLANE_FOUR_STEP_SPLIT)
+    plane4_inv_as<true>(cg, grid, nx, ny, nz, ax, ay, red, lds, s);
+  else
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
 // Batched: items are (system, first plane), plane4_group planes each (fewer at
 // the top of the grid); NT = kPlaneBlock / 2 for systems whose plane fits half
 // the LDS budget, two workgroups per CU.
-template <int INV, int NT>
+template <int INV, int NT, bool SPLIT>
 __global__ __launch_bounds__(NT, 4) void k_batch_plane4(const SysDesc* __restrict__ sys,
                                                         const WorkItem* __restrict__ items, int nitems, int reduce,
                                                         int maxnp) {
@@ -643,27 +813,36 @@ __global__ __launch_bounds__(NT, 4) void k_batch_plane4(const SysDesc* __restric
     const int np = min(plane4_group(d.bin.nx, d.bin.ny, maxnp, NT < kPlaneBlock), d.bin.nz - w.idx);
     if (INV) {
       if (reduce && w.idx == 0 && (d.sa.calc_ev || d.calc_self)) batch_ev_reduce<NT>(d);
-      plane4_inv_body<NT>(d.cgrid, d.grid, d.bin.nx, d.bin.ny, d.ax[0], d.ax[1], w.idx, np, sm);
+      plane4_inv_body<NT, SPLIT>(d.cgrid, d.grid, d.bin.nx, d.bin.ny, d.ax[0], d.ax[1], w.idx, np, sm);
     } else {
-      plane4_fwd_body<NT>(d.grid, d.cgrid, d.bin.nx, d.bin.ny, d.ax[0], d.ax[1], w.idx, np, sm);
+      plane4_fwd_body<NT, SPLIT>(d.grid, d.cgrid, d.bin.nx, d.bin.ny, d.ax[0], d.ax[1], w.idx, np, sm);
     }
     __syncthreads();
   }
 }
 
-hipError_t launch_batch_plane4(int inverse, int reduce, int maxnp, int half, const SysDesc* sys, const WorkItem* items,
-                               int nitems, int grid, size_t lds, hipStream_t s) {
-  if (nitems <= 0) return hipSuccess;
-  if (maxnp < 1 || maxnp > kPlaneGroupMax) return hipErrorInvalidValue;
+template <bool SPLIT>
+static void batch_plane4_as(int inverse, int reduce, int maxnp, int half, const SysDesc* sys, const WorkItem* items,
+                            int nitems, int grid, size_t lds, hipStream_t s) {
   constexpr int F = kPlaneBlock, H = kPlaneBlock / 2;
   if (inverse && half)
-    hipLaunchKernelGGL((k_batch_plane4<1, H>), dim3(grid), dim3(H), lds, s, sys, items, nitems, reduce, maxnp);
+    hipLaunchKernelGGL((k_batch_plane4<1, H, SPLIT>), dim3(grid), dim3(H), lds, s, sys, items, nitems, reduce, maxnp);
   else if (inverse)
-    hipLaunchKernelGGL((k_batch_plane4<1, F>), dim3(grid), dim3(F), lds, s, sys, items, nitems, reduce, maxnp);
+    hipLaunchKernelGGL((k_batch_plane4<1, F, SPLIT>), dim3(grid), dim3(F), lds, s, sys, items, nitems, reduce, maxnp);
   else if (half)
-    hipLaunchKernelGGL((k_batch_plane4<0, H>), dim3(grid), dim3(H), lds, s, sys, items, nitems, reduce, maxnp);
+    hipLaunchKernelGGL((k_batch_plane4<0, H, SPLIT>), dim3(grid), dim3(H), lds, s, sys, items, nitems, reduce, maxnp);
   else
-    hipLaunchKernelGGL((k_batch_plane4<0, F>), dim3(grid), dim3(F), lds, s, sys, items, nitems, reduce, maxnp);
+    hipLaunchKernelGGL((k_batch_plane4<0, F, SPLIT>), dim3(grid), dim3(F), lds, s, sys, items, nitems, reduce, maxnp);
+}
+
+hipError_t launch_batch_plane4(int inverse, int reduce, int maxnp, int split, int half, const SysDesc* sys,
+                               const WorkItem* items, int nitems, int grid, size_t lds, hipStream_t s) {
+  if (nitems <= 0) return hipSuccess;
+  if (maxnp < 1 || maxnp > kPlaneGroupMax) return hipErrorInvalidValue;
+  if (split)
+    batch_plane4_as<true>(inverse, reduce, maxnp, half, sys, items, nitems, grid, lds, s);
+  else
+    batch_plane4_as<false>(inverse, reduce, maxnp, half, sys, items, nitems, grid, lds, s);
   return hipGetLastError();
 }
 

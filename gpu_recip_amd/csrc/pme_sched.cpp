@@ -231,10 +231,10 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
       const SysDesc& d = *descs[k];
       const SystemPlan& p = *plans[k];
       if ((stage == BS_SPREAD || stage == BS_GATHER) && orders[k] != order) continue;
-      if (stage == BS_PLANE && (d.plane == PLANE_FOUR_STEP) != (split == 2)) continue;
-      if (stage == BS_FFTY || (stage == BS_PLANE && split != 2) || stage == BS_FFTZ) {
+      if (stage == BS_PLANE && plane_is_four_step(d.plane) != (split >= 2)) continue;
+      if (stage == BS_FFTY || stage == BS_PLANE || stage == BS_FFTZ) {
         const int a = stage == BS_FFTZ ? 2 : 1;
-        if ((d.ax[a].prec != PME_PREC_FP32) != (split != 0)) continue;
+        if ((d.ax[a].prec != PME_PREC_FP32) != ((split & 1) != 0)) continue;
       }
       // z: order 1 + c takes the systems with a four-step pair of register
       // class c, order 0 the others (Stockham stages, split precision)
@@ -267,7 +267,7 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
           break;
         case BS_PLANE: {
           if (d.plane == PLANE_NONE) break;
-          const bool f4 = d.plane == PLANE_FOUR_STEP;
+          const bool f4 = plane_is_four_step(d.plane);
           const int nx = d.bin.nx, ny = d.bin.ny, nf = d.ax[0].rp.n;
           if ((f4 ? plane4_fits_half(nx, ny) : plane_fits_half(nx, ny, nf)) != (half != 0)) break;
           const int g = f4 ? plane4_group_host(nx, ny, order, half != 0) : plane_group_host(nx, ny, nf, order, half != 0);
@@ -294,7 +294,7 @@ void build_items(const SysDesc* const* descs, const SystemPlan* const* plans, co
   for (int o : {4, 6, 8}) add_stage(BS_SPREAD, o, 0, 0);
   add_stage(BS_FFTX, 0, 0, 0);
   for (int sp : {0, 1}) add_stage(BS_FFTY, 0, sp, 0);
-  for (int sp : {0, 1, 2})
+  for (int sp : {0, 1, 2, 3})
     for (int h : {1, 0}) add_stage(BS_PLANE, group, sp, h);
   for (int c : {1, 2, 3}) add_stage(BS_FFTZ, c, 0, 0);
   for (int sp : {0, 1}) add_stage(BS_FFTZ, 0, sp, 0);
@@ -346,8 +346,8 @@ pme_status enqueue_stages(const std::vector<Launch>& launches, const SysDesc* d_
                                         stream));
             break;
           case BS_PLANE:
-            if (L.split == 2) {
-              SCHED_HIP(launch_batch_plane4(inv ? 1 : 0, inv ? 1 : 0, L.order, L.half, d_sys, it, L.count, grid, L.lds,
+            if (L.split >= 2) {
+              SCHED_HIP(launch_batch_plane4(inv ? 1 : 0, inv ? 1 : 0, L.order, L.split & 1, L.half, d_sys, it, L.count, grid, L.lds,
                                             stream));
               break;
             }

@@ -74,8 +74,8 @@ struct Launch {
   int stage;   // BatchStage
   int order;   // spread/gather template order; largest plane group of a plane launch; z pass: 1 + the
                // four-step register class, 0 for the Stockham / split kernels (0 otherwise)
-  int split;   // FFT launches: 1 for the kernels with the split-precision matrix-core stage; plane
-               // launches: 2 for the register four-step planes
+  int split;   // FFT launches: bit 0 for the kernels with the split-precision matrix-core stage; plane
+               // launches: bit 1 for the register four-step planes
   int half;    // plane launches: 1 for half-size workgroups (two per CU)
   int offset;
   int count;
