@@ -605,6 +605,25 @@ __device__ __forceinline__ void fft_cols_body(float2* __restrict__ cg, int n, in
     cols_four_step_dispatch<MODE == COL_FWD ? -1 : 1>(ax.f4col, cg, hx, TX, pt_stride, outer_stride, ax, tx, ty, sm);
     return;
   }
+  // the fused z pass of a split-precision axis of 16 f4b points
+  if constexpr (MODE == COL_FWD_SOLVE_INV && SPLIT) {
+    if (ax.prec != PREC_FP32 && ax.rp.f4a == 16) {
+      switch (ax.rp.f4b) {
+#define PME_ZS_SPLIT(L)                                                                                           \
+  case L:                                                                                                         \
+    if (ax.prec == PREC_BF16X3)                                                                                   \
+      zsolve_four_step_split<L, PREC_BF16X3>(cg, hx, TX, pt_stride, outer_stride, ax, sa, tx, ty, blk, sm, hxd);  \
+    else                                                                                                          \
+      zsolve_four_step_split<L, PREC_FP16X3>(cg, hx, TX, pt_stride, outer_stride, ax, sa, tx, ty, blk, sm, hxd);  \
+    break;
+        PME_ZS_SPLIT(2) PME_ZS_SPLIT(3) PME_ZS_SPLIT(4) PME_ZS_SPLIT(5) PME_ZS_SPLIT(6)
+        PME_ZS_SPLIT(8) PME_ZS_SPLIT(9) PME_ZS_SPLIT(10) PME_ZS_SPLIT(12) PME_ZS_SPLIT(16)
+#undef PME_ZS_SPLIT
+        default: break;
+      }
+      return;
+    }
+  }
   __shared__ double sh_red[7 * (kBlock / 64)];
   const int tid = threadIdx.x;
   float2* tw = sm;

@@ -346,6 +346,44 @@ __device__ __forceinline__ float2 solve_line_tric(const SolveArgs& s, const Line
   return cscale(q, eterm);
 }
 
+// Middle pass of the register four-step z pass: forward second half, influence
+// function, inverse first half.  Unit (l, k1), in place on the N2 points (k1 N2 +
+// j2) of b; lines kx0 + l of the flattened (ky, kx), rows of hxd.
+template <int N1, int N2, bool TRIC>
+__device__ __forceinline__ void zsolve_middle(float2* __restrict__ b, const float2* __restrict__ tw, int ts, int TX,
+                                              int kx0, int nl, int hxd, const SolveArgs& sa, double* acc) {
+  const int tsh = __builtin_ctz(TX);
+  for (int u = threadIdx.x; u < N1 * TX; u += kBlock) {
+    const int k1 = (u >> tsh);
+    const int l = u - k1 * TX;
+    float2 X[N2];
+#pragma unroll
+    for (int j2 = 0; j2 < N2; j2++) X[j2] = b[(k1 * N2 + j2) * TX + l];
+    DftN<N2, -1>::run(X);  // X[k2]: point k3 = k1 + N1 k2
+    if (l < nl) {
+      const int ky = sdiv(kx0 + l, small_div(hxd));
+      if constexpr (TRIC) {
+        const LineTric f = line_tric(sa, kx0 + l - ky * hxd, ky);
+#pragma unroll
+        for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_tric(sa, f, k1 + N1 * k2, X[k2], acc);
+      } else {
+        const LineFactors f = line_factors(sa, kx0 + l - ky * hxd, ky);
+        double sums[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+        for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_point(sa, f, k1 + N1 * k2, X[k2], sums);
+        if (sa.calc_ev) fold_line_sums(f, sums, acc);
+      }
+    }
+    DftN<N2, +1>::run(X);  // X[j2]
+#pragma unroll
+    for (int j2 = 0; j2 < N2; j2++) {
+      const float2 t = tw[mul24(j2 * k1, ts)];
+      const float2 z = j2 == 0 ? X[0] : cmul(X[j2], make_float2(t.x, -t.y));
+      b[(k1 * N2 + j2) * TX + l] = z;
+    }
+  }
+}
+
 // One column tile of the z pass (as fft_cols_body<COL_FWD_SOLVE_INV>) with
 // n = N1 N2: TX consecutive lines c0 .. c0+TX-1 of the flattened (ky, kx)
 // index of a z plane (rows of hxd), point j of line l at base + j pt_stride
@@ -395,38 +433,8 @@ __device__ __forceinline__ void zsolve_four_step(float2* __restrict__ cg, int hx
     }
   }
   __syncthreads();
-  // forward second half, influence function, inverse first half: unit (l, k1),
-  // in place on the N2 points (k1 N2 + j2) of b
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int u = tid; u < N1 * TX; u += kBlock) {
-    const int k1 = (u >> tsh);
-    const int l = u - k1 * TX;
-    float2 X[N2];
-#pragma unroll
-    for (int j2 = 0; j2 < N2; j2++) X[j2] = b[(k1 * N2 + j2) * TX + l];
-    DftN<N2, -1>::run(X);  // X[k2]: point k3 = k1 + N1 k2
-    if (l < nl) {
-      const int ky = sdiv(kx0 + l, small_div(hxd));
-      if constexpr (TRIC) {
-        const LineTric f = line_tric(sa, kx0 + l - ky * hxd, ky);
-#pragma unroll
-        for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_tric(sa, f, k1 + N1 * k2, X[k2], acc);
-      } else {
-        const LineFactors f = line_factors(sa, kx0 + l - ky * hxd, ky);
-        double sums[5] = {0, 0, 0, 0, 0};
-#pragma unroll
-        for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_point(sa, f, k1 + N1 * k2, X[k2], sums);
-        if (sa.calc_ev) fold_line_sums(f, sums, acc);
-      }
-    }
-    DftN<N2, +1>::run(X);  // X[j2]
-#pragma unroll
-    for (int j2 = 0; j2 < N2; j2++) {
-      const float2 t = tw[mul24(j2 * k1, ts)];
-      const float2 z = j2 == 0 ? X[0] : cmul(X[j2], make_float2(t.x, -t.y));
-      b[(k1 * N2 + j2) * TX + l] = z;
-    }
-  }
+  zsolve_middle<N1, N2, TRIC>(b, tw, ts, TX, kx0, nl, hxd, sa, acc);
   __syncthreads();
   // inverse second half: unit (l, j2), stored straight to HBM
   for (int u = tid; u < N2 * TX; u += kBlock) {
@@ -442,6 +450,56 @@ __device__ __forceinline__ void zsolve_four_step(float2* __restrict__ cg, int hx
       for (int j1 = 0; j1 < N1; j1++) store_through(&tile[o + (unsigned)(N2 * j1) * pst], z[j1]);
     }
   }
+  if (sa.calc_ev) ev_partial(sa, acc, sh_red, blk);
+}
+
+// The same tile for a split-precision z axis of n = 16 N2: the 16-point DFTs, which
+// are the passes that touch HBM, as hi-lo products on the matrix cores, 32 units
+// (line l, j2) per wave, lanes along l.
+template <int N2, int PREC>
+__device__ __forceinline__ void zsolve_four_step_split(float2* __restrict__ cg, int hx, int TX, long long pt_stride,
+                                                       long long outer_stride, const AxisArgs& ax,
+                                                       const SolveArgs& sa, int tx, int ty, int blk, float2* sm,
+                                                       int hxd) {
+  __shared__ double sh_red[7 * (kBlock / 64)];
+  const int tid = threadIdx.x;
+  float2* tw = sm;
+  float2* b = sm + ax.ntw;
+  for (int i = tid; i < ax.ntw; i += kBlock) tw[i] = ax.tw[i];
+  const int ts = ax.rp.tstride;
+  const int kx0 = tx * TX;
+  const int nl = min(TX, hx - kx0);
+  float2* __restrict__ tile = cg + ((size_t)kx0 + (size_t)ty * (size_t)outer_stride);
+  const unsigned pst = (unsigned)pt_stride;
+  const int tsh = __builtin_ctz(TX);
+  struct Unit {
+    unsigned o;  // point j2 of the line
+    float2* p;   // its place in b
+    int j2;
+    bool live;
+  };
+  auto unit = [&](int u) {
+    const int j2 = u >> tsh, l = u - j2 * TX;
+    return Unit{(unsigned)j2 * pst + (unsigned)l, b + (j2 * TX + l), j2, l < nl};
+  };
+  __syncthreads();  // twiddles in LDS
+  mfma_dft16_cols<-1, PREC>(
+      N2 * TX, unit,
+      [&](const Unit& x, int m) { return x.live ? tile[x.o + (unsigned)(N2 * m) * pst] : make_float2(0.f, 0.f); },
+      [&](const Unit& x, int k1, float2 y) {
+        x.p[k1 * N2 * TX] = k1 == 0 ? y : cmul(y, tw[mul24(x.j2 * k1, ts)]);
+      },
+      tid, kBlock);
+  __syncthreads();
+  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  zsolve_middle<16, N2, false>(b, tw, ts, TX, kx0, nl, hxd, sa, acc);
+  __syncthreads();
+  mfma_dft16_cols<+1, PREC>(
+      N2 * TX, unit, [&](const Unit& x, int m) { return x.p[m * N2 * TX]; },
+      [&](const Unit& x, int j1, float2 y) {
+        if (x.live) store_through(&tile[x.o + (unsigned)(N2 * j1) * pst], y);
+      },
+      tid, kBlock);
   if (sa.calc_ev) ev_partial(sa, acc, sh_red, blk);
 }
 
