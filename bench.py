@@ -41,12 +41,22 @@ PLANE_LDS_BUDGET = 150 * 1024
 
 
 def plane_mode(nfft):
-    """Whether the library runs the x and y passes of this grid as one xy
-    plane kernel: the same LDS test as fft_plane_lds_bytes (pme_fft.hip)."""
+    """Whether the library runs the x and y passes of this grid as one xy plane
+    kernel: the LDS tests of fft_plane4_lds_bytes (pme_plane.hip: both line
+    lengths products of two codelet lengths, one buffer) and, for other lengths,
+    fft_plane_lds_bytes (pme_fft.hip: two buffers)."""
     nx, ny = nfft[0], nfft[1]
-    nf = nx // 2 if nx % 2 == 0 else nx
+    even = nx % 2 == 0
+    nf = nx // 2 if even else nx
+    hx = nx // 2 + 1
+    codelets = (2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16)
+    pair = lambda n, top=16: any(a * b == n and min(a, b) <= top for a in codelets for b in codelets)  # noqa: E731
+    col = hx * (ny | 1)
+    one = col if even else nx * (((ny + 1) // 2) | 1) + col
+    if pair(nf) and pair(ny, 12) and 8 * (nx + ny + one) <= PLANE_LDS_BUDGET:
+        return True
     odd = lambda n: (n + 1) | 1  # noqa: E731
-    buf = max(nf * odd(ny), ny * odd(nx // 2 + 1))
+    buf = max(nf * odd(ny), ny * odd(hx))
     return 8 * (nx + ny + 2 * buf) <= PLANE_LDS_BUDGET
 
 
@@ -74,9 +84,9 @@ def stage_bytes(s):
 # (order 4, full bricks, every xy plane fitting a half-size plane workgroup,
 # every z length a four-step pair of register class 0)
 BATCH_KERNELS = {"bin": ("pme::k_batch_bin",), "spread": ("void pme::k_batch_spread<4, 1024>",),
-                 "fft_fwd_x_or_xy": ("void pme::k_batch_plane<0, false, 512>",),
+                 "fft_fwd_x_or_xy": ("void pme::k_batch_plane4<0, 512, false>",),
                  "fft_z_solve": ("void pme::k_batch_zsolve<0>",),
-                 "fft_inv_y_or_xy": ("void pme::k_batch_plane<1, false, 512>",),
+                 "fft_inv_y_or_xy": ("void pme::k_batch_plane4<1, 512, false>",),
                  "gather": ("void pme::k_batch_gather<4, 1024>",)}
 
 
@@ -411,7 +421,8 @@ def main():
                 # complex point per pass; the y passes run one pass, the fused
                 # z pass two (forward and inverse)
                 gc4 = (s4.nfft[0] // 2 + 1) * s4.nfft[1] * s4.nfft[2]
-                passes = {"fft_fwd_y": 1, "fft_z_solve": 2, "fft_inv_y_or_xy": 1}
+                fwd = "fft_fwd_x_or_xy" if plane_mode(s4.nfft) else "fft_fwd_y"
+                passes = {fwd: 1, "fft_z_solve": 2, "fft_inv_y_or_xy": 1}
                 mf = {}
                 for st_name, npass in passes.items():
                     fl = 384.0 * gc4 * npass
