@@ -23,9 +23,8 @@
 // go to the caller's force array as integer atomics, the j sums after every
 // pass and the i sums when the entry changes, and the shift forces of the
 // virial are summed the same way: none of these depends on the order of the
-// pairs.  Energies are per-lane FP64 sums over a fixed set of pairs, summed
-// per workgroup in wave order; a parallel fixed-order reduction adds the
-// workgroups' partials to the energy/virial buffer.
+// pairs.  Pair energies are summed as 2^32 fixed point; a parallel fixed-order
+// reduction adds the workgroups' partials to the energy/virial buffer.
 #include "pme_internal.hpp"
 
 namespace pme {
