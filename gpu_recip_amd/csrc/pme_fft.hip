@@ -605,25 +605,6 @@ __device__ __forceinline__ void fft_cols_body(float2* __restrict__ cg, int n, in
     cols_four_step_dispatch<MODE == COL_FWD ? -1 : 1>(ax.f4col, cg, hx, TX, pt_stride, outer_stride, ax, tx, ty, sm);
     return;
   }
-  // the fused z pass of a split-precision axis of 16 f4b points
-  if constexpr (MODE == COL_FWD_SOLVE_INV && SPLIT) {
-    if (ax.prec != PREC_FP32 && ax.rp.f4a == 16) {
-      switch (ax.rp.f4b) {
-#define PME_ZS_SPLIT(L)                                                                                           \
-  case L:                                                                                                         \
-    if (ax.prec == PREC_BF16X3)                                                                                   \
-      zsolve_four_step_split<L, PREC_BF16X3>(cg, hx, TX, pt_stride, outer_stride, ax, sa, tx, ty, blk, sm, hxd);  \
-    else                                                                                                          \
-      zsolve_four_step_split<L, PREC_FP16X3>(cg, hx, TX, pt_stride, outer_stride, ax, sa, tx, ty, blk, sm, hxd);  \
-    break;
-        PME_ZS_SPLIT(2) PME_ZS_SPLIT(3) PME_ZS_SPLIT(4) PME_ZS_SPLIT(5) PME_ZS_SPLIT(6)
-        PME_ZS_SPLIT(8) PME_ZS_SPLIT(9) PME_ZS_SPLIT(10) PME_ZS_SPLIT(12) PME_ZS_SPLIT(16)
-#undef PME_ZS_SPLIT
-        default: break;
-      }
-      return;
-    }
-  }
   __shared__ double sh_red[7 * (kBlock / 64)];
   const int tid = threadIdx.x;
   float2* tw = sm;
@@ -729,7 +710,8 @@ hipError_t launch_fft_cols(int mode, float2* cg, int n, int hx, int TX, long lon
                            int hxd, hipStream_t s) {
   const bool split = ax.prec != PREC_FP32;
   const bool four_step = mode == COL_FWD_SOLVE_INV && !split && ax.f4 >= 0;
-  const size_t lds = fft_cols_lds_bytes(n, TX, four_step ? 1 : 2);
+  const bool split_four_step = mode == COL_FWD_SOLVE_INV && split && ax.rp.f4a == 16;
+  const size_t lds = fft_cols_lds_bytes(n, TX, four_step || split_four_step ? 1 : 2);
   const dim3 grid((hx + TX - 1) / TX, nouter);
   // the fused z pass indexes its tile with shifts
   if (mode == COL_FWD_SOLVE_INV && sa.tric && !four_step) return hipErrorInvalidValue;  // no such kernel
@@ -737,6 +719,10 @@ hipError_t launch_fft_cols(int mode, float2* cg, int n, int hx, int TX, long lon
   if (four_step) {
     if (nouter != 1 || outer_stride != 0) return hipErrorInvalidValue;  // one flattened plane of lines
     return launch_zsolve(cg, hx, TX, pt_stride, ax, sa, red, hxd, lds, s);
+  }
+  if (split_four_step) {
+    if (nouter != 1 || outer_stride != 0) return hipErrorInvalidValue;
+    return launch_zsolve_split(cg, hx, TX, pt_stride, ax, sa, red, hxd, lds, s);
   }
 #define PME_COLS(M)                                                                                         \
   if (split)                                                                                              \
@@ -781,8 +767,30 @@ __global__ __launch_bounds__(kBlock) void k_batch_fft_x(const SysDesc* __restric
   }
 }
 
+// the fused z pass of a split-precision axis of 16 f4b points (a single
+// system's: k_zsolve_split)
+__device__ __forceinline__ void zsolve_split_dispatch(float2* __restrict__ cg, int hx, int TX, long long pt_stride,
+                                                      const AxisArgs& ax, const SolveArgs& sa, int blk, float2* sm,
+                                                      int hxd) {
+  switch (ax.rp.f4b) {
+#define PME_ZS_SPLIT(L)                                                                                  \
+  case L:                                                                                                \
+    if (ax.prec == PREC_BF16X3)                                                                          \
+      zsolve_four_step_split<L, PREC_BF16X3>(cg, hx, TX, pt_stride, 0, ax, sa, blk, 0, blk, sm, hxd);    \
+    else                                                                                                 \
+      zsolve_four_step_split<L, PREC_FP16X3>(cg, hx, TX, pt_stride, 0, ax, sa, blk, 0, blk, sm, hxd);    \
+    break;
+    PME_ZSOLVE_SPLIT_LENGTHS(PME_ZS_SPLIT)
+#undef PME_ZS_SPLIT
+    default: break;
+  }
+}
+
+// split z passes: held to three waves per SIMD (the compiler takes 256 VGPRs
+// for the union of the lengths, one wave).  24 systems of 48 to 96 points, planes
+// included: 286 -> 207 us per solve.
 template <int AXIS, int MODE, bool SPLIT>
-__global__ __launch_bounds__(kBlock) void k_batch_cols(const SysDesc* __restrict__ sys,
+__global__ __launch_bounds__(kBlock, AXIS == 2 && SPLIT ? 3 : 1) void k_batch_cols(const SysDesc* __restrict__ sys,
                                                        const WorkItem* __restrict__ items, int nitems, int reduce) {
   extern __shared__ __align__(16) float2 sm[];
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
@@ -795,6 +803,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_cols(const SysDesc* __restrict
       const int ntx = (hx + d.TXy - 1) / d.TXy;
       fft_cols_body<MODE, SPLIT>(d.cgrid, d.bin.ny, hx, d.TXy, hx, pz, d.ax[1], d.sa, w.idx % ntx, w.idx / ntx,
                                  w.idx, sm, hx);
+    } else if (SPLIT && MODE == COL_FWD_SOLVE_INV && d.ax[2].rp.f4a == 16 && d.ax[2].prec != PREC_FP32) {
+      zsolve_split_dispatch(d.cgrid, hx * d.bin.ny, d.TXz, pz, d.ax[2], d.sa, w.idx, sm, hx);
     } else {  // z: tiles of the flattened (ky, kx) of a plane
       fft_cols_body<MODE, SPLIT>(d.cgrid, d.bin.nz, hx * d.bin.ny, d.TXz, pz, 0, d.ax[2], d.sa, w.idx, 0, w.idx, sm,
                                  hx);

@@ -244,6 +244,8 @@ hipError_t launch_fft_cols(int mode, float2* cg, int n, int hx, int TX, long lon
                            const SolveArgs& sa, const EvReduce& red, int hxd, hipStream_t s);
 int cols_blocks(int hx, int TX, int nouter);
 // the fused z pass of a length with a four-step pair (pme_zsolve.hip), sa.tric included
+hipError_t launch_zsolve_split(float2* cg, int nlines, int TX, long long pt_stride, const AxisArgs& ax,
+                               const SolveArgs& sa, const EvReduce& red, int hxd, size_t lds, hipStream_t s);
 hipError_t launch_zsolve(float2* cg, int nlines, int TX, long long pt_stride, const AxisArgs& ax, const SolveArgs& sa,
                          const EvReduce& red, int hxd, size_t lds, hipStream_t s);
 // every point of the half spectrum times f

@@ -453,6 +453,9 @@ __device__ __forceinline__ void zsolve_four_step(float2* __restrict__ cg, int hx
   if (sa.calc_ev) ev_partial(sa, acc, sh_red, blk);
 }
 
+// N2 of the split-precision z lengths 16 N2 (radix_plan_split)
+#define PME_ZSOLVE_SPLIT_LENGTHS(X) X(2) X(3) X(4) X(5) X(6) X(8) X(9) X(10) X(12) X(16)
+
 // The same tile for a split-precision z axis of n = 16 N2: the 16-point DFTs, which
 // are the passes that touch HBM, as hi-lo products on the matrix cores, 32 units
 // (line l, j2) per wave, lanes along l.
