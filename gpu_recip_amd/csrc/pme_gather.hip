@@ -192,7 +192,7 @@ __device__ __forceinline__ void gather_brick_body(const float4* __restrict__ xyz
       atom[r] = -1;
       pos[r] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (v < total) {
-        const size_t slot = brick_record(a, v, s_pre, s_base);
+        const RecordSlot slot = brick_record(a, v, s_pre, s_base);
         atom[r] = a.rec_idx[slot];
         if (FROM_REC) pos[r] = a.rec_pos[slot];
       }

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/pme_recip.h"
+#include "pme_slots.hpp"
 #include "pme_device.hpp"
 
 namespace pme {
@@ -208,14 +209,14 @@ __device__ __forceinline__ int xcd_brick(int blk, int nbricks) {
 }
 
 // record slot of the v-th record of the brick (0 <= v < total)
-__device__ __forceinline__ size_t brick_record(const BinArgs& a, int v, const int* s_pre, const int* s_base) {
+__device__ __forceinline__ RecordSlot brick_record(const BinArgs& a, int v, const int* s_pre, const int* s_base) {
   int lo = 0, hi = a.nchunk;  // s_pre[lo] <= v < s_pre[hi]
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (s_pre[mid] <= v) lo = mid;
     else hi = mid;
   }
-  return (size_t)lo * a.rec_stride + s_base[lo] + (v - s_pre[lo]);
+  return record_slot(lo, a.rec_stride, s_base[lo] + (v - s_pre[lo]));
 }
 
 // ---- launchers (return the HIP error of the launch) ----

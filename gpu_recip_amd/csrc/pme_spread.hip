@@ -370,7 +370,6 @@ __device__ __forceinline__ void store_brick_pairs(const unsigned long long* __re
   }
 }
 
-constexpr size_t kNoSlot = (size_t)-1;
 // Orders 6 and 8 only: at 4 a record has too few stencil points for the sort to
 // pay (250k atoms, 144^3: 19.7 against 19.2 us; 64-system set 65.7 against 59.2 us).
 template <int P> constexpr bool kBankOrder = P >= 6;
@@ -384,7 +383,8 @@ template <int P> constexpr bool kBankOrder = P >= 6;
 // sorted list, spreads the lanes of a wave over the banks.  The list holds
 // record slots.  Integer sums do not depend on the order.
 template <int NT>
-__device__ __forceinline__ size_t bank_order(size_t slot, int bank, bool on, int nbat, int* s_cnt, int* s_list) {
+__device__ __forceinline__ RecordSlot bank_order(RecordSlot slot, int bank, bool on, int nbat, int* s_cnt,
+                                                 RecordList* s_list) {
   const int tid = threadIdx.x, lane = tid & 63;
   int rank = 0;
   if (on) rank = atomicAdd(&s_cnt[bank], 1);
@@ -397,12 +397,12 @@ __device__ __forceinline__ size_t bank_order(size_t slot, int bank, bool on, int
     if ((lane & 31) >= off) v += t;
   }
   const int start = __shfl(v - cnt, bank, 32);
-  if (on) s_list[start + rank] = (int)slot;
+  if (on) s_list[start + rank] = slot;
   __syncthreads();
   if (tid < 32) s_cnt[tid] = 0;  // for the next batch
   const int R = (nbat + 31) >> 5;
   const int at = mul24(tid & 31, R) + (tid >> 5);
-  return (tid >> 5) < R && at < nbat ? (size_t)s_list[at] : kNoSlot;
+  return (tid >> 5) < R && at < nbat ? s_list[at] : kNoSlot;
 }
 
 // Brick b of one grid (one NT-thread workgroup); smem: the workgroup's
@@ -415,7 +415,7 @@ __device__ __forceinline__ void spread_brick_body(const BinArgs& a, int b, int w
                                                   float* __restrict__ grid, unsigned char* smem) {
   __shared__ int sh_scan[NT / 64];
   __shared__ int s_cnt[32];
-  __shared__ int s_list[NT];
+  __shared__ RecordList s_list[NT];
 
   const int bxs = spread_xstride(wxm, P);
   unsigned long long* acc = reinterpret_cast<unsigned long long*>(smem);
@@ -441,7 +441,7 @@ __device__ __forceinline__ void spread_brick_body(const BinArgs& a, int b, int w
     const int nbat = min(NT, total - base);
     const bool on = tid < nbat;
     if (kBankOrder<P>) {
-      size_t slot = on ? brick_record(a, base + tid, s_pre, s_base) : kNoSlot;
+      RecordSlot slot = on ? brick_record(a, base + tid, s_pre, s_base) : kNoSlot;
       float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
       if (on) p = a.rec_pos[slot];
       int ix, iy, iz;
