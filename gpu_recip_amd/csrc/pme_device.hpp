@@ -473,7 +473,10 @@ __device__ __forceinline__ void mfma_dft16_cols(int ncols, Prep prep, Load load,
       for (int t = 0; t < 8; t++) mx = fmaxf(mx, fmaxf(fabsf(x[t].x), fabsf(x[t].y)));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       if (mx > 0.0f) {
-        const int ex = ilogbf(mx);
+        // below 2^-114 the scale itself would overflow (columns near both Nyquist
+        // edges, after the influence function): the smallest exponent whose scale
+        // is finite, 2^127; such a column stays below the others' rounding
+        const int ex = max(ilogbf(mx), -114);
         scale = ldexpf(1.0f, 13 - ex);
         unscale = ldexpf(1.0f, ex - 13);
       }
