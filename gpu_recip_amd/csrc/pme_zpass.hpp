@@ -346,6 +346,25 @@ __device__ __forceinline__ float2 solve_line_tric(const SolveArgs& s, const Line
   return cscale(q, eterm);
 }
 
+// Influence function over the N2 points k3 = k1 + N1 k2 (X[k2]) of line `line` of
+// the flattened (ky, kx), rows of hxd
+template <int N1, int N2, bool TRIC>
+__device__ __forceinline__ void solve_line_points(const SolveArgs& sa, float2* X, int k1, int line, int hxd,
+                                                  double* acc) {
+  const int ky = sdiv(line, small_div(hxd));
+  if constexpr (TRIC) {
+    const LineTric f = line_tric(sa, line - ky * hxd, ky);
+#pragma unroll
+    for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_tric(sa, f, k1 + N1 * k2, X[k2], acc);
+  } else {
+    const LineFactors f = line_factors(sa, line - ky * hxd, ky);
+    double sums[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+    for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_point(sa, f, k1 + N1 * k2, X[k2], sums);
+    if (sa.calc_ev) fold_line_sums(f, sums, acc);
+  }
+}
+
 // Middle pass of the register four-step z pass: forward second half, influence
 // function, inverse first half.  Unit (l, k1), in place on the N2 points (k1 N2 +
 // j2) of b; lines kx0 + l of the flattened (ky, kx), rows of hxd.
@@ -360,20 +379,7 @@ __device__ __forceinline__ void zsolve_middle(float2* __restrict__ b, const floa
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) X[j2] = b[(k1 * N2 + j2) * TX + l];
     DftN<N2, -1>::run(X);  // X[k2]: point k3 = k1 + N1 k2
-    if (l < nl) {
-      const int ky = sdiv(kx0 + l, small_div(hxd));
-      if constexpr (TRIC) {
-        const LineTric f = line_tric(sa, kx0 + l - ky * hxd, ky);
-#pragma unroll
-        for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_tric(sa, f, k1 + N1 * k2, X[k2], acc);
-      } else {
-        const LineFactors f = line_factors(sa, kx0 + l - ky * hxd, ky);
-        double sums[5] = {0, 0, 0, 0, 0};
-#pragma unroll
-        for (int k2 = 0; k2 < N2; k2++) X[k2] = solve_line_point(sa, f, k1 + N1 * k2, X[k2], sums);
-        if (sa.calc_ev) fold_line_sums(f, sums, acc);
-      }
-    }
+    if (l < nl) solve_line_points<N1, N2, TRIC>(sa, X, k1, kx0 + l, hxd, acc);
     DftN<N2, +1>::run(X);  // X[j2]
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) {
@@ -456,9 +462,18 @@ __device__ __forceinline__ void zsolve_four_step(float2* __restrict__ cg, int hx
 // N2 of the split-precision z lengths 16 N2 (radix_plan_split)
 #define PME_ZSOLVE_SPLIT_LENGTHS(X) X(2) X(3) X(4) X(5) X(6) X(8) X(9) X(10) X(12) X(16)
 
-// The same tile for a split-precision z axis of n = 16 N2: the 16-point DFTs, which
-// are the passes that touch HBM, as hi-lo products on the matrix cores, 32 units
-// (line l, j2) per wave, lanes along l.
+// The same tile for a split-precision z axis of n = 16 N2: the 16-point DFTs as
+// hi-lo products on the matrix cores, 32 units per wave, lanes along l.  They come
+// first in both directions: the hi-lo error goes with the largest value of a
+// 16-point column, and behind the other factor a column of the inverse mixes large
+// and small frequencies (250,002 atoms, 144^3, BF16x3: forces 3.83e-5 from FP64 that
+// way with one LDS exchange less and 20.9 us, 3.79e-5 this way in 23.1 us; FP32 transforms
+// 3.48e-5).  So the inverse splits k = k2 + N2 k1, j = j1 + 16 j2, and
+// the buffer holds the spectrum in natural order between the two:
+//   1  HBM -> DFT_16 over j1 of j2 + N2 j1, twiddle -> slot k1 + 16 j2
+//   2  slots k1 + 16 j2 -> DFT_N2, influence function -> slot k3 = k1 + 16 k2, in place
+//   3  slots k2 + N2 k1 -> DFT_16 over k1, twiddle -> slot k2 + N2 j1, in place
+//   4  slots k2 + N2 j1 -> DFT_N2 -> HBM, points j1 + 16 j2
 template <int N2, int PREC>
 __device__ __forceinline__ void zsolve_four_step_split(float2* __restrict__ cg, int hx, int TX, long long pt_stride,
                                                        long long outer_stride, const AxisArgs& ax,
@@ -476,33 +491,55 @@ __device__ __forceinline__ void zsolve_four_step_split(float2* __restrict__ cg, 
   const unsigned pst = (unsigned)pt_stride;
   const int tsh = __builtin_ctz(TX);
   struct Unit {
-    unsigned o;  // point j2 of the line
-    float2* p;   // its place in b
-    int j2;
+    unsigned o;  // point q of the line
+    int l, q;
     bool live;
   };
   auto unit = [&](int u) {
-    const int j2 = u >> tsh, l = u - j2 * TX;
-    return Unit{(unsigned)j2 * pst + (unsigned)l, b + (j2 * TX + l), j2, l < nl};
+    const int q = u >> tsh, l = u - q * TX;
+    return Unit{(unsigned)q * pst + (unsigned)l, l, q, l < nl};
   };
   __syncthreads();  // twiddles in LDS
   mfma_dft16_cols<-1, PREC>(
       N2 * TX, unit,
       [&](const Unit& x, int m) { return x.live ? tile[x.o + (unsigned)(N2 * m) * pst] : make_float2(0.f, 0.f); },
       [&](const Unit& x, int k1, float2 y) {
-        x.p[k1 * N2 * TX] = k1 == 0 ? y : cmul(y, tw[mul24(x.j2 * k1, ts)]);
+        b[(k1 + 16 * x.q) * TX + x.l] = k1 == 0 ? y : cmul(y, tw[mul24(x.q * k1, ts)]);
       },
       tid, kBlock);
   __syncthreads();
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  zsolve_middle<16, N2, false>(b, tw, ts, TX, kx0, nl, hxd, sa, acc);
+  for (int u = tid; u < 16 * TX; u += kBlock) {
+    const int k1 = u >> tsh, l = u - k1 * TX;
+    float2 X[N2];
+#pragma unroll
+    for (int j2 = 0; j2 < N2; j2++) X[j2] = b[(k1 + 16 * j2) * TX + l];
+    DftN<N2, -1>::run(X);
+    if (l < nl) solve_line_points<16, N2, false>(sa, X, k1, kx0 + l, hxd, acc);
+#pragma unroll
+    for (int k2 = 0; k2 < N2; k2++) b[(k1 + 16 * k2) * TX + l] = X[k2];
+  }
   __syncthreads();
   mfma_dft16_cols<+1, PREC>(
-      N2 * TX, unit, [&](const Unit& x, int m) { return x.p[m * N2 * TX]; },
+      N2 * TX, unit, [&](const Unit& x, int m) { return b[(x.q + N2 * m) * TX + x.l]; },
       [&](const Unit& x, int j1, float2 y) {
-        if (x.live) store_through(&tile[x.o + (unsigned)(N2 * j1) * pst], y);
+        const float2 t = tw[mul24(x.q * j1, ts)];
+        b[(x.q + N2 * j1) * TX + x.l] = j1 == 0 ? y : cmul(y, make_float2(t.x, -t.y));
       },
       tid, kBlock);
+  __syncthreads();
+  for (int u = tid; u < 16 * TX; u += kBlock) {
+    const int j1 = u >> tsh, l = u - j1 * TX;
+    float2 X[N2];
+#pragma unroll
+    for (int k2 = 0; k2 < N2; k2++) X[k2] = b[(k2 + N2 * j1) * TX + l];
+    DftN<N2, +1>::run(X);
+    if (l < nl) {
+      const unsigned o = (unsigned)j1 * pst + (unsigned)l;
+#pragma unroll
+      for (int j2 = 0; j2 < N2; j2++) store_through(&tile[o + (unsigned)(16 * j2) * pst], X[j2]);
+    }
+  }
   if (sa.calc_ev) ev_partial(sa, acc, sh_red, blk);
 }
 

@@ -75,7 +75,7 @@ hipError_t launch_zsolve(float2* cg, int nlines, int TX, long long pt_stride, co
 }
 
 // The split-precision z pass of one grid, one kernel per length and precision
-// (144^3, BF16x3: 20.9 us; 23.5 as one kernel for all of them, three waves per SIMD).
+// (one kernel for all of them takes 2.6 us more at 144^3, three waves per SIMD).
 template <int N2, int PREC>
 __global__ __launch_bounds__(kBlock, 4) void k_zsolve_split(float2* __restrict__ cg, int nlines, int TX,
                                                             long long pt_stride, AxisArgs ax, SolveArgs sa,
