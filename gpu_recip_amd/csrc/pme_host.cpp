@@ -260,6 +260,7 @@ struct pme_recip_s {
 
   // bricks and the chunked record store of the binning
   int nb[3] = {1, 1, 1}, wmax[3] = {0, 0, 0}, nbins = 0;
+  BrickPlan lean = {};        // fewer bricks: a solve in the static scratch that the plan above does not fit
   int ncu = 256;              // compute units of the device
   int bins_for = -1;          // atom capacity of the record store
   int chunk = 0, nchunk = 0, nchunk_cap = 0;
@@ -378,6 +379,14 @@ static pme_status upload_prefac(pme_recip_t h) {
   return PME_OK;
 }
 
+static void use_bricks(pme_recip_t h, const BrickPlan& bp) {
+  for (int a = 0; a < 3; a++) {
+    h->nb[a] = bp.nb[a];
+    h->wmax[a] = bp.wmax[a];
+  }
+  h->nbins = bp.nbins;
+}
+
 static bool plan_bricks(pme_recip_t h) {
   const int n[3] = {h->nx, h->ny, h->nz};
   BrickPlan bp;
@@ -386,11 +395,8 @@ static bool plan_bricks(pme_recip_t h) {
       hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || h->ncu <= 0)
     h->ncu = 256;
   if (!pme::plan_bricks_auto(n, h->order, h->ncu, &bp)) return false;
-  for (int a = 0; a < 3; a++) {
-    h->nb[a] = bp.nb[a];
-    h->wmax[a] = bp.wmax[a];
-  }
-  h->nbins = bp.nbins;
+  if (!pme::plan_bricks_auto(n, h->order, h->ncu, &h->lean, true)) h->lean = bp;
+  use_bricks(h, bp);
   return true;
 }
 
@@ -990,13 +996,13 @@ static pme_status scratch_address(void** out) {
   return PME_OK;
 }
 
-// Offsets of the work buffers of an n-atom solve in the scratch array
-// (256-byte aligned); returns the bytes used.
+// Offsets of the work buffers of an n-atom solve with nbins bricks in the scratch
+// array (256-byte aligned); returns the bytes used.
 struct ScratchLayout {
   size_t grid, cgrid, seg_off, rec_pos, rec_idx, partial, total;
   int chunk, nchunk;
 };
-static ScratchLayout scratch_layout(pme_recip_t h, int n) {
+static ScratchLayout scratch_layout(pme_recip_t h, int n, int nbins) {
   ScratchLayout L{};
   const ChunkPlan cp = plan_chunks(n);
   L.chunk = cp.chunk;
@@ -1011,7 +1017,7 @@ static ScratchLayout scratch_layout(pme_recip_t h, int n) {
   };
   L.grid = take(sizeof(float) * G);
   L.cgrid = take(sizeof(float2) * (size_t)spec_pitch(h->nx / 2 + 1, h->ny) * h->nz);
-  L.seg_off = take(sizeof(int) * (size_t)cp.nchunk * seg_stride(h->nbins));
+  L.seg_off = take(sizeof(int) * (size_t)cp.nchunk * seg_stride(nbins));
   L.rec_pos = take(sizeof(float4) * rs);
   L.rec_idx = take(sizeof(int) * rs);
   L.partial = take(sizeof(double) * 7 * (size_t)h->partial_cap);
@@ -1026,7 +1032,15 @@ extern "C" pme_status pme_recip_solve_noalloc(pme_recip_t h, const void* d_xyzq,
   if (ncoord < 0) return fail(PME_ERR_INVALID_ARG, "pme_recip_solve_noalloc: ncoord %d", ncoord);
   if (!box_ok(recip))
     return fail(PME_ERR_INVALID_ARG, "pme_recip_solve_noalloc: recip has no positive determinant");
-  const ScratchLayout L = scratch_layout(h, ncoord);
+  // the handle's brick plan, or the one with fewer bricks where only that fits (the
+  // results do not depend on the bricks)
+  ScratchLayout L = scratch_layout(h, ncoord, h->nbins);
+  BrickPlan bp{{h->nb[0], h->nb[1], h->nb[2]}, {h->wmax[0], h->wmax[1], h->wmax[2]}, h->nbins};
+  const BrickPlan own = bp;
+  if (L.total > kScratchBytes) {
+    bp = h->lean;
+    L = scratch_layout(h, ncoord, bp.nbins);
+  }
   if (L.total > kScratchBytes)
     return fail(PME_ERR_BUDGET,
                 "pme_recip_solve_noalloc: %d atoms on a %dx%dx%d grid need %zu bytes of work buffers, "
@@ -1050,6 +1064,7 @@ extern "C" pme_status pme_recip_solve_noalloc(pme_recip_t h, const void* d_xyzq,
   h->rec_pos = reinterpret_cast<float4*>(base + L.rec_pos);
   h->rec_idx = reinterpret_cast<int*>(base + L.rec_idx);
   h->partial = reinterpret_cast<double*>(base + L.partial);
+  use_bricks(h, bp);
   // the record store is sized for exactly this call, so the binning never reallocates
   h->chunk = L.chunk;
   h->nchunk = h->nchunk_cap = L.nchunk;
@@ -1066,6 +1081,7 @@ extern "C" pme_status pme_recip_solve_noalloc(pme_recip_t h, const void* d_xyzq,
   h->rec_pos = rec_pos;
   h->rec_idx = rec_idx;
   h->partial = partial;
+  use_bricks(h, own);
   h->bins_for = bins_for;
   h->chunk = chunk;
   h->nchunk = nchunk;

@@ -169,11 +169,15 @@ static double brick_cost(const int n[3], int order, int ncu, const BrickPlan& bp
 // gather 17.3 -> 16.2).  Targets below 16 are for grids with fewer bricks of 16
 // than CUs (23,559 atoms, 64^3, order 6, 64 -> 252 bricks: spread 17.6 -> 13.6, gather
 // 12.2 -> 9.6; 2,001 atoms, 32^3, order 4, 8 -> 64 bricks: 7.7 -> 6.3, 6.9 -> 5.9).
-bool plan_bricks_auto(const int n[3], int order, int ncu, BrickPlan* bp) {
+// lean: targets from 16 up and cubic counts only, for a fixed scratch: more bricks
+// lengthen the segment table of every chunk (64^3, order 6, 380,000 atoms: 0.19 MB with
+// 64 bricks, 0.75 MB with 252).
+bool plan_bricks_auto(const int n[3], int order, int ncu, BrickPlan* bp, bool lean) {
   bool any = false;
   double best = 0.0;
   for (int target : {8, 10, 12, 14, 16, 18, 20, 24, 28, 32})
     for (int more = 0; more < 4; more++) {
+      if (lean && (target < 16 || more > 0)) continue;
       BrickPlan t;
       const int extra[3] = {0, more >> 1, more & 1};
       if (!plan_bricks(n, order, target, &t, kBrickLdsBudget, extra)) continue;

@@ -46,8 +46,9 @@ struct BrickPlan {
 bool plan_bricks(const int n[3], int order, int target, BrickPlan* bp, size_t budget = kBrickLdsBudget,
                  const int* extra = nullptr);
 // The brick plan of a single-system solve on ncu CUs: of the plans for brick
-// targets 8 to 32, the one with the least modelled spread time per CU
-bool plan_bricks_auto(const int n[3], int order, int ncu, BrickPlan* bp);
+// targets 8 to 32 (lean: fewer, larger bricks), the one with the least modelled
+// spread time per CU
+bool plan_bricks_auto(const int n[3], int order, int ncu, BrickPlan* bp, bool lean = false);
 
 struct FftTiles {
   int NR, TXy, TXz;
