@@ -23,8 +23,9 @@
 // go to the caller's force array as integer atomics, the j sums after every
 // pass and the i sums when the entry changes, and the shift forces of the
 // virial are summed the same way: none of these depends on the order of the
-// pairs.  Pair energies are summed as 2^32 fixed point; a parallel fixed-order
-// reduction adds the workgroups' partials to the energy/virial buffer.
+// pairs.  Pair energies are summed as 2^32 fixed point.  Which workgroup takes which
+// tiles varies from run to run, so the workgroups' partials stay integers until
+// one reduction has added them all and converts the sum once.
 #include "pme_internal.hpp"
 
 namespace pme {
@@ -399,14 +400,15 @@ __global__ __launch_bounds__(kDirWaves * 64) void k_direct_force(DirectParams d,
   if (ENERGY || VIRIAL) {
     if (ENERGY && pot != 0) atomicAdd(&s_pot, (unsigned long long)pot);
     __syncthreads();
-    double* out = partial + blockIdx.x;
+    // integers in the partials' places (k_direct_reduce<true>)
+    long long* out = reinterpret_cast<long long*>(partial) + blockIdx.x;
     const size_t st = gridDim.x;
     const int tid = threadIdx.x;
     if (ENERGY && tid == 0) {
-      out[0] = (double)(long long)s_pot * (1.0 / 4294967296.0);
-      out[st] = 0.0;
+      out[0] = (long long)s_pot;
+      out[st] = 0;
     }
-    if (VIRIAL && tid < 81) out[(2 + tid) * st] = (double)(long long)s_sf[tid] * (1.0 / 1099511627776.0);
+    if (VIRIAL && tid < 81) out[(2 + tid) * st] = (long long)s_sf[tid];
   }
 }
 
@@ -452,10 +454,39 @@ __global__ __launch_bounds__(kDir14Block) void k_direct_14(DirectParams d, int n
                                       partial + blockIdx.x, gridDim.x);
 }
 
-// Sum the partials of nblk workgroups (slot c of workgroup b at c nblk + b) and add them into the energy/virial
-// buffer: the elec and excl slots and sforce_dp[27][3].  One workgroup per
-// slot; thread k sums workgroups k, k + 256, ... and block_sum adds the
-// threads in fixed order (the same result on every run).
+// Sum of the 64-bit integers v[0], v[1], ... v[n-1] times scale, rounded once: the
+// high and the low halves are summed apart, so no total overflows (256 threads; the
+// result in thread 0).
+__device__ __forceinline__ double block_sum_fixed(const long long* __restrict__ v, int n, double scale) {
+  __shared__ unsigned long long s_half[2];
+  if (threadIdx.x < 2) s_half[threadIdx.x] = 0ull;
+  __syncthreads();
+  long long hi = 0, lo = 0;
+  for (int b = threadIdx.x; b < n; b += 256) {
+    hi += v[b] >> 32;
+    lo += v[b] & 0xffffffffll;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    hi += __shfl_xor(hi, off, 64);
+    lo += __shfl_xor(lo, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(&s_half[0], (unsigned long long)hi);
+    atomicAdd(&s_half[1], (unsigned long long)lo);
+  }
+  __syncthreads();
+  const long long h = (long long)s_half[0] + (long long)(s_half[1] >> 32);
+  return __fma_rn((double)h, 4294967296.0 * scale, (double)(unsigned)s_half[1] * scale);
+}
+
+// Sum the partials of nblk workgroups (slot c of workgroup b at c nblk + b) and add
+// them into the energy/virial buffer: the elec and excl slots and
+// sforce_dp[27][3].  One workgroup per slot.  FIXED: the pair kernel's integers
+// (energies 2^32, shift forces 2^40 fixed point), whose sum does not depend on the
+// order; else FP64 values, thread k summing workgroups k, k + 256, ... and
+// block_sum the threads in fixed order.  The same result on every run either way.
+template <bool FIXED>
 __global__ __launch_bounds__(256) void k_direct_reduce(const double* __restrict__ partial, int nblk, int energy,
                                                        int virial, double* e_elec, double* e_excl,
                                                        double* sforce_dp) {
@@ -463,8 +494,13 @@ __global__ __launch_bounds__(256) void k_direct_reduce(const double* __restrict_
   const int c = blockIdx.x;
   if ((c < 2 && !energy) || (c >= 2 && !virial)) return;
   double acc = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += 256) acc += partial[(size_t)c * nblk + b];
-  block_sum<1, 256>(&acc, s_red);
+  if (FIXED) {
+    acc = block_sum_fixed(reinterpret_cast<const long long*>(partial) + (size_t)c * nblk, nblk,
+                          c < 2 ? 1.0 / 4294967296.0 : 1.0 / 1099511627776.0);
+  } else {
+    for (int b = threadIdx.x; b < nblk; b += 256) acc += partial[(size_t)c * nblk + b];
+    block_sum<1, 256>(&acc, s_red);
+  }
   if (threadIdx.x == 0) {
     if (c == 0) e_elec[0] += acc;
     else if (c == 1) e_excl[0] += acc;
@@ -516,11 +552,15 @@ hipError_t launch_direct_14(const DirectParams& d, int nin14, int nex14, const p
   return hipGetLastError();
 }
 
-hipError_t launch_direct_reduce(const double* partial, int nblk, bool energy, bool virial, double* e_elec,
+hipError_t launch_direct_reduce(bool fixed, const double* partial, int nblk, bool energy, bool virial, double* e_elec,
                                 double* e_excl, double* sforce_dp, hipStream_t s) {
   if (nblk == 0 || !(energy || virial)) return hipSuccess;
-  hipLaunchKernelGGL(k_direct_reduce, dim3(kDirPartial), dim3(256), 0, s, partial, nblk, energy ? 1 : 0,
-                     virial ? 1 : 0, e_elec, e_excl, sforce_dp);
+  const dim3 g(kDirPartial), b(256);
+  const int ce = energy ? 1 : 0, cv = virial ? 1 : 0;
+  if (fixed)
+    hipLaunchKernelGGL(k_direct_reduce<true>, g, b, 0, s, partial, nblk, ce, cv, e_elec, e_excl, sforce_dp);
+  else
+    hipLaunchKernelGGL(k_direct_reduce<false>, g, b, 0, s, partial, nblk, ce, cv, e_elec, e_excl, sforce_dp);
   return hipGetLastError();
 }
 

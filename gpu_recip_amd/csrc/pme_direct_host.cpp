@@ -218,7 +218,7 @@ extern "C" pme_status pme_direct_calc_14_force(pme_direct_t h, const void* d_xyz
   if (ce || cv) PME_TRY(ensure_partial(h, nblk, s));
   HIP_TRY(launch_direct_14(h->d, h->nin14, h->nex14, h->in14, h->ex14, (const float4*)d_xyzq, stride,
                            reinterpret_cast<unsigned long long*>(d_force), ce, cv, h->partial, s));
-  HIP_TRY(launch_direct_reduce(h->partial, nblk, ce, cv, h->e_elec, h->e_excl, h->sforce_dp, s));
+  HIP_TRY(launch_direct_reduce(false, h->partial, nblk, ce, cv, h->e_elec, h->e_excl, h->sforce_dp, s));
   return PME_OK;
 }
 
@@ -251,6 +251,6 @@ extern "C" pme_status pme_direct_calc_force(pme_direct_t h, const void* d_xyzq, 
                               h->tile_entry + kDirQueueInts,
                               nlist->tile_indj, nlist->tile_excl, (const float4*)d_xyzq, stride,
                               reinterpret_cast<unsigned long long*>(d_force), ce, cv, h->partial, s));
-  HIP_TRY(launch_direct_reduce(h->partial, nblk, ce, cv, h->e_elec, h->e_excl, h->sforce_dp, s));
+  HIP_TRY(launch_direct_reduce(true, h->partial, nblk, ce, cv, h->e_elec, h->e_excl, h->sforce_dp, s));
   return PME_OK;
 }

@@ -443,8 +443,9 @@ hipError_t launch_direct_force(const DirectParams& d, int n_ientry, int n_tile, 
 hipError_t launch_direct_14(const DirectParams& d, int nin14, int nex14, const pme_xx14* in14, const pme_xx14* ex14,
                             const float4* xyzq, int stride, unsigned long long* force, bool energy, bool virial,
                             double* partial, hipStream_t s);
-// adds the nblk partials (fixed order) to the elec / excl terms and sforce_dp[27][3]
-hipError_t launch_direct_reduce(const double* partial, int nblk, bool energy, bool virial, double* e_elec,
+// adds the nblk partials to the elec / excl terms and sforce_dp[27][3]; fixed: those
+// of the pair kernel, 64-bit fixed point
+hipError_t launch_direct_reduce(bool fixed, const double* partial, int nblk, bool energy, bool virial, double* e_elec,
                                 double* e_excl, double* sforce_dp, hipStream_t s);
 int direct_force_blocks(int nwave);
 int direct_force_waves(int n_tile, int ncu);
