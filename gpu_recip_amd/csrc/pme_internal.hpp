@@ -416,7 +416,8 @@ constexpr int kPlaneBlock = 1024;   // threads per xy plane FFT workgroup
 constexpr int kPlaneGroupMax = 4;   // z planes per batched plane workgroup (at most)
 constexpr size_t kPlaneLdsBudget = 150 * 1024;  // the plane kernels run one workgroup per CU at most
 constexpr int kMaxChunks = 512;    // binning workgroups per solve (chunk grows with n)
-static_assert(kMaxChunks <= kSpreadBlock, "brick_segments: one thread per chunk");
+// the half-size workgroups of the spread and gather too
+static_assert(kMaxChunks <= kSpreadBlock / 2, "brick_segments: one thread per chunk");
 constexpr int kMinChunk = 512;    // atoms per binning workgroup
 
 
