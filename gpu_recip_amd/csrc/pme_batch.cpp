@@ -4,7 +4,8 @@
 // energy/virial partials stay resident in HBM, admission is checked against
 // the batch's HBM budget.  A solve of a subset of slots runs the same stage
 // bodies as the single-system solver, but every stage is ONE launch over all
-// systems (persistent workgroups walking a per-stage work list), and the
+// systems over a per-stage work list (one workgroup per brick in spread and gather;
+// one per item, or persistent ones walking the list, in the others), and the
 // whole 8-launch sequence is captured once in a hipGraph and replayed while
 // the subset and the launch shapes stay the same.  Coordinates, box and
 // outputs are read from the device descriptor table at run time, so updating

@@ -5,27 +5,27 @@
 // CudaDirectForceKernels.cu:352-400, 506-716).
 //
 // Non-bonded pairs.  The waves take the list's j tiles two at a time from a few
-// queues as they finish, so the waves' loads even
-// out whatever the spread of the tiles' pair counts; a small kernel first maps
-// every j tile to its entry.
-// Each half of a wave takes one tile per pass, one j atom per lane, holding the i tile of the tile's entry (32 atoms, moved by
-// the entry's periodic shift on the j side) in LDS and flushing the i-force
-// sums whenever the entry changes.  A pass has two phases.  The check phase
-// tests the 32 x 64 pairs against the cutoff, each lane reading the i atoms
-// at LDS addresses common to its half (broadcast reads) and building a 32-bit
-// mask of its interacting i atoms; the tile's exclusion words, rotated into
-// the same bit order, clear the excluded pairs.  The dense phase packs the
-// wave's interacting pairs into an LDS queue (bit round by bit round, each round a
-// ballot, so that 64 consecutive pairs belong to different j atoms) and evaluates
-// them 64 at a time, so the Ewald term runs only for pairs inside the cutoff (about one check in eight
-// for a 32-atom tile list).  Pair forces are rounded once to 2^40 fixed
-// point and summed with integer LDS atomics per i and per j atom; the sums
-// go to the caller's force array as integer atomics, the j sums after every
-// pass and the i sums when the entry changes, and the shift forces of the
-// virial are summed the same way: none of these depends on the order of the
-// pairs.  Pair energies are summed as 2^32 fixed point.  Which workgroup takes which
-// tiles varies from run to run, so the workgroups' partials stay integers until
-// one reduction has added them all and converts the sum once.
+// queues as they finish, so the waves' loads even out whatever the spread of the
+// tiles' pair counts; a small kernel first maps every j tile to its entry.  Each
+// half of a wave takes one tile per pass, one j atom per lane, holding the i tile
+// of the tile's entry (32 atoms, moved by the entry's periodic shift on the j
+// side) in LDS and flushing the i-force sums whenever the entry changes (with
+// tiles from a queue, on most passes).  A pass has two phases.  The check phase
+// tests the 32 x 64 pairs against the cutoff, each lane reading the i atoms at LDS
+// addresses common to its half (broadcast reads) and building a 32-bit mask of
+// its interacting i atoms; rotated into the bit order of the tile's exclusion
+// words, the mask loses the excluded pairs.  The dense phase packs the wave's
+// interacting pairs into an LDS queue (bit round by bit round, each round a ballot,
+// so that 64 consecutive pairs belong to different j atoms) and evaluates them 64 at
+// a time, so the Ewald term runs only for pairs inside the cutoff (about one check
+// in eight for a 32-atom tile list).  Pair forces are rounded once to 2^40 fixed
+// point and summed with integer LDS atomics per i and per j atom; the sums go to
+// the caller's force array as integer atomics, the j sums after every pass and the
+// i sums when the entry changes, and the shift forces of the virial are summed the
+// same way: none of these depends on the order of the pairs.  Pair energies are
+// summed as 2^32 fixed point.  Which workgroup takes which tiles varies from run to
+// run, so the workgroups' partials stay integers until one reduction has added them
+// all and converts the sum once.
 #include "pme_internal.hpp"
 
 namespace pme {

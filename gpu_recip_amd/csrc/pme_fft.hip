@@ -787,7 +787,7 @@ __device__ __forceinline__ void zsolve_split_dispatch(float2* __restrict__ cg, i
 }
 
 // split z passes: held to three waves per SIMD (the compiler takes 256 VGPRs
-// for the union of the lengths, one wave).  24 systems of 48 to 96 points, planes
+// for the union of the lengths, one wave; 22 are spilled).  24 systems of 48 to 96 points, planes
 // included: 286 -> 207 us per solve (211 with the 16-point DFT first in the inverse).
 template <int AXIS, int MODE, bool SPLIT>
 __global__ __launch_bounds__(kBlock, AXIS == 2 && SPLIT ? 3 : 1) void k_batch_cols(const SysDesc* __restrict__ sys,

@@ -256,8 +256,10 @@ hipError_t launch_gather(int order, int force_type, const float4* xyzq, const Bi
 
 // NT = kSpreadBlock / 2: half-size workgroups for bricks planned within half the
 // LDS budget.  The gather's halo brick is about half of the spread's, so three
-// share a CU when the registers allow (12 instead of 24 halo loads in flight:
-// 80 VGPRs at order 4): 64-system set 46.1 -> 40.8 us.
+// share a CU when the registers allow (12 instead of 24 halo loads in flight; 67
+// VGPRs at order 4, and 80 at order 6, where the bound of six waves per SIMD spills
+// seven): order 4, 64-system set 46.1 -> 40.8 us; order 6, whole solves of the same 64
+// systems 351 us at six waves, 359 at five and 364 at four, without spills.
 template <int P, int NT>
 __global__ __launch_bounds__(NT, NT < kSpreadBlock && P < 8 ? 6 : 4) void k_batch_gather(const SysDesc* __restrict__ sys,
                                                      const WorkItem* __restrict__ items) {

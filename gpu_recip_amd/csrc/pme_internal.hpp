@@ -381,7 +381,8 @@ hipError_t launch_batch_plane4(int inverse, int reduce, int maxnp, int split, in
 // how the x and y passes of a grid run (y_prec: PREC_* of the y axis)
 PlaneKind plane_kind(int nx, int ny, const RadixPlan& rx, const RadixPlan& ry, int y_prec);
 
-// batched launchers: `grid` persistent workgroups loop over the work items
+// batched launchers: `grid` workgroups loop over the work items (spread and gather:
+// one per item)
 hipError_t launch_batch_bin(const SysDesc* sys, const WorkItem* items, int nitems, int grid, size_t lds, hipStream_t s);
 // spread / gather: half != 0 runs kSpreadBlock / 2 threads per workgroup
 // (bricks planned within half the LDS budget, two workgroups per CU)

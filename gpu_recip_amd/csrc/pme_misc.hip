@@ -30,7 +30,7 @@ hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s) {
 // workgroup, after a reduction still pending on it: one launch in place of a
 // reduction kernel and a copy command, whose set-up and completion cost more
 // than the bytes (23,559 atoms, 64^3, order 6, self energy, read back every
-// solve: 120 -> 102 us).  red writes into dev, so no restrict here.
+// solve: 119 -> 114 us).  red writes into dev, so no restrict here.
 __global__ __launch_bounds__(kBlock) void k_copy_out(unsigned long long* host, const unsigned long long* dev,
                                                      int nwords, EvReduce red) {
   ev_reduce_block<kBlock>(red);

@@ -801,7 +801,8 @@ hipError_t launch_plane4_inv(const float2* cg, float* grid, int nx, int ny, int 
 
 // Batched: items are (system, first plane), plane4_group planes each (fewer at
 // the top of the grid); NT = kPlaneBlock / 2 for systems whose plane fits half
-// the LDS budget, two workgroups per CU.
+// the LDS budget, two workgroups per CU.  Held to 128 VGPRs (four waves per SIMD),
+// where the inverse spills one VGPR in FP32 and three in split precision.
 template <int INV, int NT, bool SPLIT>
 __global__ __launch_bounds__(NT, 4) void k_batch_plane4(const SysDesc* __restrict__ sys,
                                                         const WorkItem* __restrict__ items, int nitems, int reduce,

@@ -2,13 +2,13 @@
 // semantics), re-designed for CDNA4:
 //
 //  1. k_bin_chunks: a chunked counting sort.  Workgroup w bins its chunk of
-//     atoms by grid brick with LDS counters only (histogram, block scan,
-//     cursors): an atom gets one record in every brick its p^3 stencil
-//     touches (1 to 8), the copy in the brick of its base index is its
+//     atoms by grid brick with LDS counters only (each count's old value is the
+//     record's rank, then a block scan): an atom gets one record in every brick its
+//     p^3 stencil touches (1 to 8), the copy in the brick of its base index is its
 //     "home" record.  No global atomics, so nothing contends across the 8 XCDs.
 //  2. k_spread_brick: one workgroup per brick.  It reads exactly the records
-//     of its brick (all of them touch it), computes the B-spline weights into
-//     LDS and accumulates q*thx*thy*thz in LDS as 64-bit fixed point with
+//     of its brick (all of them touch it), one per thread with the B-spline
+//     weights in registers, and accumulates q*thx*thy*thz in LDS as 64-bit fixed point with
 //     scale 2^40 -- the reference's `long long` grid accumulation
 //     (CudaPMERecip.cu:51-58, write_grid<long long>; reduce_force, reduce.cu:66-78).
 //     Integer LDS atomics are an order of magnitude faster than float ones

@@ -230,9 +230,9 @@ __device__ __forceinline__ void ev_partial(const SolveArgs& s, double* acc, doub
 // the largest single pair (all 31 pairs and the Stockham stages: 157 VGPRs,
 // three waves per SIMD; one pair: 72 to 118).  The batched z pass therefore
 // has one kernel per class: class 0 holds the pairs with N2 <= 10 and 5 x 15
-// (75, a common edge; held to 128 VGPRs, four waves per SIMD, with three
+// (75, a common edge; held to 128 VGPRs, four waves per SIMD, with five
 // spilled), class 1 the pairs up to 12 x 16 (125 VGPRs), class 2 those with a longer
-// codelet (not held to 128).
+// codelet (153 VGPRs, not held to 128).
 constexpr int f4_class_of(int n1, int n2) {
   return (n2 <= 10 || (n1 == 5 && n2 == 15)) ? 0 : (n2 <= 16 ? 1 : 2);
 }

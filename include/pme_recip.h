@@ -188,7 +188,7 @@ pme_status pme_fill_bspline(int order, int nfftx, int nffty, int nfftz,
 
 /* ---------------- batched path (no counterpart in the reference) ----------------
  * Many independent orthorhombic systems solved together: every stage is one
- * launch over all systems (persistent workgroups over per-stage work lists),
+ * launch over all systems (workgroups over per-stage work lists),
  * and the whole sequence is captured once in a hipGraph and replayed.  Each
  * system keeps its grids, FFT plans and binning store resident in HBM
  * ("slots"); admission is checked against the HBM budget of the batch.
